@@ -31,6 +31,7 @@ DEVICE = ["-x", "hip", "--offload-arch=" + ARCH,
 
 SOURCES = [
     ("march.hip", True),
+    ("line.hip", True),
     ("voxel.hip", True),
     ("batch.hip", True),
     ("surrogate.hip", True),

@@ -537,6 +537,121 @@ bool compose_linear(const std::vector<xrp::HDeform>& defs, double M[9], double t
   return true;
 }
 
+// Whether the interval march (line_march.hpp) takes a scene, and with what:
+// the object-space map must be affine and well conditioned, and the tree one
+// primitive, a collection of them, or a tessellation of a collection of
+// convex ones.  Gyroids of a collection contribute runs found by their safe
+// reach, so they must be wide: at most about two periods along a ray.
+// Steps under 1e-5 (ten times the roots' FP32 error) and degenerate
+// primitives stay with the sampling marches.  $XRP_INTERVALS=0 turns the
+// march off, and the switches that choose among the sampling marches (XRP_TWO_PASS,
+// XRP_BLOCK, XRP_QUEUE, XRP_TILE, read per render) imply that.
+bool line_plan(const xrp::Scene& s, const RenderJob& job, double lip, double s_err,
+               xrp::MarchParams& mp) {
+  using namespace xrp;
+  const char* e = std::getenv("XRP_INTERVALS");
+  if (e && std::strcmp(e, "0") == 0) return false;
+  for (const char* name : {"XRP_TWO_PASS", "XRP_BLOCK", "XRP_QUEUE", "XRP_TILE"})
+    if (std::getenv(name)) return false;
+  if (!skip_enabled() || !cull_enabled() || !reach_enabled()) return false;
+  double M[9], t[3];
+  if (!compose_linear(s.defs, M, t)) return false;
+  const double unit = job.integrator == XRP_INTEGRATE_HIERARCHICAL ? job.ds / 10.0 : job.ds;
+  if (!(unit >= 1e-5)) return false;
+  // condition number (Frobenius) of the map
+  const double det = M[0] * (M[4] * M[8] - M[5] * M[7]) - M[1] * (M[3] * M[8] - M[5] * M[6]) +
+                     M[2] * (M[3] * M[7] - M[4] * M[6]);
+  double f2 = 0, c2 = 0;
+  for (int k = 0; k < 9; ++k) f2 += M[k] * M[k];
+  for (int r = 0; r < 3; ++r)
+    for (int c = 0; c < 3; ++c) {
+      const int r1 = (r + 1) % 3, r2 = (r + 2) % 3, c1 = (c + 1) % 3, c3 = (c + 2) % 3;
+      const double m = M[3 * r1 + c1] * M[3 * r2 + c3] - M[3 * r1 + c3] * M[3 * r2 + c1];
+      c2 += m * m;
+    }
+  const double cond = std::sqrt(f2 * c2) / std::fabs(det);
+  if (!(cond < 1e4) || !std::isfinite(f2)) return false;
+  // object-space reach of a ray from the origin
+  double W = std::sqrt(f2) * (2.0 * std::fabs(job.R) + kCubeHalfDiagonal);
+  for (int k = 0; k < 3; ++k) W += std::fabs(t[k]);
+  const HNode& root = s.root;
+  const bool tess = root.kind == K_TESS;
+  if (tess && (root.kids.size() != 1 || root.kids[0].kind != K_COLL)) return false;
+  const HNode* kids = &root;
+  size_t n_kids = 1, gyroids = 0;
+  if (tess || root.kind == K_COLL) {
+    const HNode& c = tess ? root.kids[0] : root;
+    kids = c.kids.data();
+    n_kids = c.kids.size();
+  }
+  if (n_kids == 0 || s.nodes.size() > 32767) return false;
+  double cell = 0.0;
+  if (tess) {
+    for (int k = 0; k < 3; ++k) {
+      const double d = root.ucb[2 * k + 1] - root.ucb[2 * k];
+      if (!(d > 0)) return false;
+      cell += std::max({d, std::fabs(root.ucb[2 * k]), std::fabs(root.ucb[2 * k + 1])});
+      if (!std::isfinite(root.bounds[2 * k]) || !std::isfinite(root.bounds[2 * k + 1])) return false;
+    }
+    if (n_kids > (size_t)kLineCellCap) return false;
+  }
+  for (size_t q = 0; q < n_kids; ++q) {
+    const HNode& n = kids[q];
+    double least = 0;
+    switch (n.kind) {
+      case K_SPHERE: least = n.a; break;
+      case K_BOX: least = std::min({n.v[0], n.v[1], n.v[2]}); break;
+      case K_PPED: {
+        // the smallest height over a face: 1 / |row of M^-1|
+        least = INFINITY;
+        for (int i = 0; i < 3; ++i)
+          least = std::min(least, 1.0 / std::sqrt(n.minv[i] * n.minv[i] +
+                                                  n.minv[3 + i] * n.minv[3 + i] +
+                                                  n.minv[6 + i] * n.minv[6 + i]));
+        break;
+      }
+      case K_CYL: {
+        double vv = 0;
+        for (int k = 0; k < 3; ++k) vv += (n.v[k] - n.c[k]) * (n.v[k] - n.c[k]);
+        least = std::min(n.a, std::sqrt(vv));
+        break;
+      }
+      case K_GYROID:
+        if (tess) return false;
+        // path length 2 * half diagonal over the period 2 pi scale
+        if (!(6.2831853 * std::fabs(n.a) >= lip * kCubeHalfDiagonal)) return false;
+        ++gyroids;
+        least = INFINITY;
+        break;
+      default: return false;
+    }
+    for (int k = 0; k < 3; ++k)
+      if (!std::isfinite(n.c[k])) return false;
+    if (!(least >= 1e-9 * W) || !std::isfinite(n.rho)) return false;
+  }
+  std::memcpy(mp.M, M, sizeof M);
+  std::memcpy(mp.t, t, sizeof t);
+  mp.line = tess ? LINE_TESS : LINE_COLL;
+  // Run slots of a collection's segment.  Few slots keep many waves resident
+  // (32: 18 one-wave workgroups per CU), too few halve the segments again
+  // and again: 60 children 0.36 ms at 32 slots, 0.39 at 64; 179 children 4.0
+  // at 48, 2.08 at 64, 2.10 at 96, 2.8 at 128.  Launches of few waves (at most four
+  // per CU) take a slot per possible run: their wide pencils of rays meet
+  // most children, and nothing competes for the LDS.
+  const size_t need = n_kids + 2 * gyroids;
+  const size_t tiles = (size_t)((job.res + 7) / 8) * (size_t)((job.res + 7) / 8) * job.views.size();
+  const size_t cap = tiles <= 1024 ? (size_t)kLineCapMost
+                     : n_kids <= 64 ? (size_t)kLineCap
+                     : n_kids <= 128 ? 2 * (size_t)kLineCap : 3 * (size_t)kLineCap;
+  mp.line_cap = tess ? (int)n_kids : (int)std::min(cap, std::max<size_t>(4, need));
+  // FP64 roundings of positions through the chain (64 ulps of the reach), the
+  // sample table's drift, and, for cells, FP32 cell-local coordinates
+  const double pos = 64.0 * 2.3e-16 * W * (1.0 + (double)s.defs.size()) + 2.0 * lip * s_err;
+  mp.line_eps = (float)(pos + (tess ? 4.0 * cell / 16777216.0 : 0.0));
+  mp.line_seam = 64.0 * pos;
+  return true;
+}
+
 // Brick-order copies of a voxel root that the voxel-root kernel reads.
 enum BrickSlot { SLOT_PLAIN = 0, SLOT_PAIR = 1, SLOT_QUAD = 2, N_SLOTS = 3 };
 
@@ -628,7 +743,7 @@ struct LaunchPlan {
 };
 
 int plan_job(xrp_context* ctx, xrp_scene* sc, const RenderJob& job, LaunchPlan& pl,
-             bool allow_voxel_kernel = true, bool no_alloc = false) {
+             bool allow_voxel_kernel = true, bool no_alloc = false, bool allow_line = false) {
   using namespace xrp;
   Scene& s = *sc->s;
   const int res = job.res;
@@ -673,9 +788,10 @@ int plan_job(xrp_context* ctx, xrp_scene* sc, const RenderJob& job, LaunchPlan& 
   } else {
     Bw = 2.0 * std::fabs(job.R) + kCubeHalfDiagonal + 1.0;
   }
-  double delta = 0.0, lipschitz = 1.0;
+  double delta = 0.0, lipschitz = 1.0, table_err = 0.0;
   if (precision == XRP_PRECISION_GUARDED && !vox_kernel) {
     double step = job.integrator == XRP_INTEGRATE_SIMPLE ? 32.0 * job.ds : 0.0;
+    table_err = (10.0 * K + 4.0) * 2.3e-16 * std::max(std::fabs(smin), std::fabs(smax));
     // simple march anchors: smin + k ds against the table's K accumulated
     // additions (each off by at most half an ulp of |s|)
     double s_err = job.integrator == XRP_INTEGRATE_SIMPLE
@@ -689,6 +805,12 @@ int plan_job(xrp_context* ctx, xrp_scene* sc, const RenderJob& job, LaunchPlan& 
     // and ran 2.8x slower than guarded.
     if (!(delta < 0.1 * s.min_feature)) precision = XRP_PRECISION_FP64;
   }
+  MarchParams line;
+  std::memset(&line, 0, sizeof line);
+  if (allow_line && precision == XRP_PRECISION_GUARDED && !vox_kernel &&
+      line_plan(s, job, lipschitz, table_err, line))
+    // its gyroids are evaluated at FP32 strides of the whole path
+    (void)compute_guards(s, Bw, 2.0 * kCubeHalfDiagonal, nullptr, table_err);
 
   std::vector<void*> vptr;
   if (s.has_voxels) {
@@ -833,6 +955,14 @@ int plan_job(xrp_context* ctx, xrp_scene* sc, const RenderJob& job, LaunchPlan& 
     // FP32 anchor rounding (u*|G|) plus the FP32 step (4u * |B| * chunk*ds).
     mp.vguard = (float)(4.0 * (u * (N + 4.0 * L * 0.5 * N * 32.0 * job.ds) + 1e-9));
   }
+  if (line.line) {
+    mp.line = line.line;
+    mp.line_cap = line.line_cap;
+    mp.line_eps = line.line_eps;
+    mp.line_seam = line.line_seam;
+    std::memcpy(mp.M, line.M, sizeof mp.M);
+    std::memcpy(mp.t, line.t, sizeof mp.t);
+  }
   pl.precision = precision;
   pl.vox_kernel = vox_kernel;
   pl.layout = layout;
@@ -854,7 +984,7 @@ int render_core(xrp_context* ctx, xrp_scene* sc, const RenderJob& job,
   const int res = job.res;
   HIPCHK(hipSetDevice(ctx->device));
   LaunchPlan pl;
-  int rc = plan_job(ctx, sc, job, pl, true, fixed != nullptr);
+  int rc = plan_job(ctx, sc, job, pl, true, fixed != nullptr, /*allow_line=*/true);
   if (rc) return rc;
   const int precision = pl.precision;
   const bool vox_kernel = pl.vox_kernel;
@@ -875,12 +1005,14 @@ int render_core(xrp_context* ctx, xrp_scene* sc, const RenderJob& job,
   // index.  Not under audit, nor without allocation.
   const int kMaxGridY = 65535;
   const bool hier = job.integrator == XRP_INTEGRATE_HIERARCHICAL;
+  const bool line = pl.mp.line != LINE_NONE;
   const bool two_pass = !fixed && !one_pass && !sc->one_pass &&
                         precision == XRP_PRECISION_GUARDED && !vox_kernel && !job.audit &&
+                        (line ? !hier && (size_t)nv * res * res >= ((size_t)1 << 21) :
                         (hier ? s.root.kind != K_COLL || two_pass_forced() : !pl.mp.queue) &&
                         (pl.mp.block == 1 || pl.mp.block == 2) &&
                         ((size_t)nv * res * res >= ((size_t)1 << 21) || two_pass_forced()) &&
-                        two_pass_enabled();
+                        two_pass_enabled());
   int vpc = two_pass ? (int)std::min<size_t>(kMaxGridY, ((size_t)1 << 31) / ((size_t)res * res))
                      : kMaxGridY;
   if (const char* e = std::getenv("XRP_LAUNCH_VIEWS"))  // fewer views per launch, for tests
@@ -1004,6 +1136,7 @@ int render_core(xrp_context* ctx, xrp_scene* sc, const RenderJob& job,
     int integ = job.integrator == XRP_INTEGRATE_HIERARCHICAL ? INT_HIERARCHICAL
                                                              : INT_SIMPLE;
     int e = vox_kernel ? launch_voxel(mp, layout, ctx->stream)
+            : line     ? launch_line(mp, integ, ctx->stream)
                        : launch_march(mp, prec, integ, ctx->stream);
     if (e != 0) {
       // the staging copy may still be reading the pinned buffer

@@ -84,6 +84,9 @@ static_assert(sizeof(DevNode) == 256, "DevNode must stay 256 bytes");
 //  TESS   f: bounds(6) ucmin(3) dx dy dz inv_dx inv_dy inv_dz
 //         d: bounds(6) ucmin(3) ucmax(3)   (dx = ucmax - ucmin, objects.go:574)
 //  VOXEL  f: (nx-1)/2 (ny-1)/2 (nz-1)/2
+//  f[13..15], interval march (line_march.hpp): SPHERE [14] r; CYL [13] axis
+//          length, [14] r; PPED [13] longest row of M^-1, [14] sum of the
+//          edges' lengths.
 //  guards: SPHERE/CYL q-band in [0]; CYL t-band in [1]; BOX/PPED per axis
 //          [0..2]; GYROID [0]; TESS wrap (fraction units) [0], bounds [1];
 //          VOXEL bounds [0]; COLL sum-near-zero band [0] (hierarchical).

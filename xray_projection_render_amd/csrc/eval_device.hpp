@@ -265,11 +265,12 @@ __device__ __forceinline__ double density64(const MarchParams& p, double x,
 // has density 0 along the wave's rays, so the sum over the list (in the
 // same order), and the result, are those of the full walk
 // (objects.go:422-438).
-__device__ __forceinline__ double density64(const MarchParams& p, double x, double y,
-                                            double z, const int16_t* idx, int n) {
-  deform64(p.defs, p.n_defs, x, y, z);
-  if (n < 0) return node64<0>(p.nodes, 0, x, y, z);
-  const DevNode* __restrict__ N = p.nodes;
+__device__ __forceinline__ double density64(const DevNode* __restrict__ N,
+                                            const DevDeform* __restrict__ defs, int n_defs,
+                                            double x, double y, double z, const int16_t* idx,
+                                            int n) {
+  deform64(defs, n_defs, x, y, z);
+  if (n < 0) return node64<0>(N, 0, x, y, z);
   const bool greedy = N[0].greedy;
   double density = 0.0;
   for (int t = 0; t < n; ++t) {
@@ -295,7 +296,10 @@ __device__ __forceinline__ double density64(const MarchParams& p, double x, doub
     density = 1.0;
   return density;
 }
-
+__device__ __forceinline__ double density64(const MarchParams& p, double x, double y,
+                                            double z, const int16_t* idx, int n) {
+  return density64(p.nodes, p.defs, p.n_defs, x, y, z, idx, n);
+}
 
 // ---------------------------------------------------------------------------
 // Guarded FP32 evaluator.  Returns the exact FP64 density when every

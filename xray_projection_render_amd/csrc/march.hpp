@@ -123,7 +123,26 @@ struct MarchParams {
   // sample's FP32 position by more than its guard band (the FP32 density
   // of a sample is then the same with or without the child).
   float cull_pad;
+  // Interval march (line_march.hpp): LINE_NONE, or the root's form.  M and t
+  // then hold the composed deformation.  line_cap: run slots per wave;
+  // line_eps: object-space bound on the FP64 position errors (both
+  // renderers') and, for cells, on the FP32 rounding of cell-local
+  // coordinates; line_seam: distance from a cell face within which an index
+  // is evaluated in FP64.
+  int32_t line;
+  int32_t line_cap;
+  float line_eps;
+  double line_seam;
 };
+
+enum LineKind : int32_t { LINE_NONE = 0, LINE_COLL = 1, LINE_TESS = 2 };
+// Slots of a collection's segment: 8.25 KiB of LDS per wave, so that 18
+// one-wave workgroups fit a CU; more runs in one segment halve it.
+constexpr int kLineCap = 32;
+// Most slots of any launch (62 KiB; more need a larger LDS opt-in).
+constexpr int kLineCapMost = 240;
+// Most children of a cell the interval march takes (one slot each).
+constexpr int kLineCellCap = 96;
 
 // Guard-band samples a ray may defer to the resolve pass (the first pass
 // keeps them in LDS: 6 KiB per wave, so that 24 one-wave workgroups, 6 per
@@ -235,6 +254,11 @@ int launch_batch_reset(uint32_t* counters, int n_counters, unsigned long long* t
 // at 0), bytes into out; res^3 entries each.
 int launch_volume(const MarchParams& p, int res, double* dens,
                   unsigned long long* maxbits, unsigned char* out, void* stream);
+
+// Interval march of every pixel (p.line != LINE_NONE).  With p.redo_list
+// (simple integrator) in two passes: rays with an index that needs the FP64
+// evaluator are appended to it, and marched again by the second.
+int launch_line(const MarchParams& p, int integrator, void* stream);
 
 // Launch on the given stream; returns hipError_t as int.
 int launch_march(const MarchParams& p, int precision, int integrator,

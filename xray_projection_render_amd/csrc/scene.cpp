@@ -727,6 +727,7 @@ void flatten(const HNode& n, int depth, std::vector<DevNode>& out, Scene& s) {
       dn.d[4] = n.rho;
       dn.f[3] = (float)(n.a * n.a);
       dn.f[4] = (float)n.rho;
+      dn.f[14] = (float)n.a;
       break;
     case K_BOX:
       for (int k = 0; k < 3; ++k) {
@@ -749,6 +750,12 @@ void flatten(const HNode& n, int depth, std::vector<DevNode>& out, Scene& s) {
       }
       dn.d[12] = n.rho;
       dn.f[12] = (float)n.rho;
+      for (int i = 0; i < 3; ++i) {  // longest row of M^-1 (column-major), edge lengths
+        const double* m = n.minv;
+        const double row = std::sqrt(m[i] * m[i] + m[3 + i] * m[3 + i] + m[6 + i] * m[6 + i]);
+        dn.f[13] = std::max(dn.f[13], (float)(row * (1 + 1e-6)));
+        dn.f[14] += (float)vlen3(n.pv + 3 * i);
+      }
       break;
     case K_CYL: {
       double v0 = n.v[0] - n.c[0], v1 = n.v[1] - n.c[1], v2 = n.v[2] - n.c[2];
@@ -770,6 +777,8 @@ void flatten(const HNode& n, int depth, std::vector<DevNode>& out, Scene& s) {
       dn.f[7] = (float)(1.0 / vv);
       dn.f[8] = (float)(n.a * n.a);
       dn.f[9] = (float)n.rho;
+      dn.f[13] = (float)(std::sqrt(vv) * (1 + 1e-6));
+      dn.f[14] = (float)n.a;
       break;
     }
     case K_GYROID:
