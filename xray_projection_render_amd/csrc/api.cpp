@@ -418,6 +418,7 @@ struct RenderJob {
   double ds, R, fov, flat_field, dm;
   int integrator, precision, audit;
   int output = 0, transparency = 0;
+  bool batched = false;  // one of many in a launch
 };
 
 size_t pixel_bytes(int output) { return output == XRP_OUTPUT_GRAY8_ALPHA8 ? 2 : 4; }
@@ -640,7 +641,7 @@ bool line_plan(const xrp::Scene& s, const RenderJob& job, double lip, double s_e
   // most children, and nothing competes for the LDS.
   const size_t need = n_kids + 2 * gyroids;
   const size_t tiles = (size_t)((job.res + 7) / 8) * (size_t)((job.res + 7) / 8) * job.views.size();
-  const size_t cap = tiles <= 1024 ? (size_t)kLineCapMost
+  const size_t cap = tiles <= 1024 && !job.batched ? (size_t)kLineCapMost
                      : n_kids <= 64 ? (size_t)kLineCap
                      : n_kids <= 128 ? 2 * (size_t)kLineCap : 3 * (size_t)kLineCap;
   mp.line_cap = tess ? (int)n_kids : (int)std::min(cap, std::max<size_t>(4, need));
@@ -1452,6 +1453,7 @@ struct xrp_batch {
   std::vector<double> cost;           // per item: estimated work per tile
   struct Group {
     int prec = 0, integ = 0;
+    bool line = false;                // interval march
     std::vector<int> items;           // queue order (smallest total work first)
     int first = 0;                    // offset of the group's jobs in `jobs`
     uint32_t n_tiles = 0;
@@ -1523,6 +1525,10 @@ void record_tuned(const std::string& sig, const xrp_tile_shape& t) {
   }
 }
 
+// One-wave workgroups of the interval march per 256-thread workgroup that
+// the tile shape counts.
+constexpr int kLineBatchWaves = 8;
+
 // Tile the queue for b->shape and capture reset + persistent launches.
 int apply_shape(xrp_batch* b) {
   using namespace xrp;
@@ -1572,7 +1578,12 @@ int apply_shape(xrp_batch* b) {
     bg.wave_rows = b->shape.wave_rows;
     bg.wave_cols = b->shape.wave_cols;
     const int wgs = std::max(1, b->n_cu * b->shape.groups_per_cu);
-    e = launch_batch(bg, g.prec, g.integ, wgs, ctx->stream);
+    if (g.line) {
+      for (int it : g.items) bg.line_cap = std::max(bg.line_cap, b->mps[it].line_cap);
+      e = launch_batch_line(bg, g.integ, kLineBatchWaves * wgs, ctx->stream);
+    } else {
+      e = launch_batch(bg, g.prec, g.integ, wgs, ctx->stream);
+    }
   }
   hipGraph_t graph = nullptr;
   hipError_t ce = hipStreamEndCapture(ctx->stream, &graph);
@@ -1675,7 +1686,9 @@ int xrp_batch_create(xrp_context* ctx, const xrp_batch_item* items, int n_items,
       xrp_scene* sc = const_cast<xrp_scene*>(items[it].scene);
       RenderJob job = make_job(&items[it].params, items[it].views, items[it].n_views);
       LaunchPlan pl;
-      int rc = plan_job(ctx, sc, job, pl, /*allow_voxel_kernel=*/false);
+      job.batched = true;
+      int rc = plan_job(ctx, sc, job, pl, /*allow_voxel_kernel=*/false, /*no_alloc=*/false,
+                        /*allow_line=*/true);
       if (rc) return rc;
       const Scene& s = *sc->s;
       node_off.push_back(all_nodes.size());
@@ -1709,7 +1722,7 @@ int xrp_batch_create(xrp_context* ctx, const xrp_batch_item* items, int n_items,
     }
     b->signature = sig;
 
-    // Groups by (precision, integrator).  Within a group the scenes are
+    // Groups by (precision, integrator, interval march).  Within a group the scenes are
     // queued whole, in order of estimated total work (work per tile x
     // pixels), smallest first: each scene then finishes as early as its
     // place allows, which minimises the mean and median completion time,
@@ -1718,13 +1731,15 @@ int xrp_batch_create(xrp_context* ctx, const xrp_batch_item* items, int n_items,
     // tile, largest first (for comparison).
     for (int it = 0; it < n_items; ++it) {
       auto g = std::find_if(b->groups.begin(), b->groups.end(), [&](const xrp_batch::Group& x) {
-        return x.prec == b->prec[it] && x.integ == b->integ[it];
+        return x.prec == b->prec[it] && x.integ == b->integ[it] &&
+               x.line == (b->mps[it].line != LINE_NONE);
       });
       if (g == b->groups.end()) {
         b->groups.push_back(xrp_batch::Group());
         g = b->groups.end() - 1;
         g->prec = b->prec[it];
         g->integ = b->integ[it];
+        g->line = b->mps[it].line != LINE_NONE;
       }
       g->items.push_back(it);
     }

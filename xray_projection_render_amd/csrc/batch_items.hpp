@@ -1,0 +1,108 @@
+// batch_items.hpp - work-queue bookkeeping shared by the batched persistent
+// kernels (batch.hip, line.hip).
+#pragma once
+#include <hip/hip_runtime.h>
+
+#include "march.hpp"
+#include "march_ray.hpp"
+
+namespace xrp {
+
+// Atomics issued by every lane of a wave: control flow stays wave-uniform
+// inside the persistent loop (no lane-conditional blocks next to the loop's
+// back edge, where a divergent branch could split one wave's lanes across
+// loop iterations; a lane-0-only form faulted for that reason).  Only the
+// first active lane targets the real address; every other lane hits a line
+// of its own in the sink, so an item costs one same-address operation per
+// counter instead of 64 (a one-scene batch of 8192 items: 3.2 us per item,
+// serialized on its scene's counters).
+__device__ __forceinline__ bool first_lane() {
+  return __builtin_amdgcn_readfirstlane((int)(threadIdx.x & 63)) == (int)(threadIdx.x & 63);
+}
+
+template <typename T>
+__device__ __forceinline__ T* lane_slot(T* real, unsigned long long* sink) {
+  return first_lane() ? real : (T*)(sink + 16 * (threadIdx.x & 63));
+}
+
+__device__ __forceinline__ void wave_add(unsigned long long* p, unsigned long long v,
+                                         unsigned long long* sink) {
+  atomicAdd(lane_slot(p, sink), first_lane() ? v : 0ull);
+}
+
+// Items a wave takes per counter operation.  A wave adds its stats and its
+// scene's last-end stamp once per run of consecutive items of one scene
+// (items are queued scene by scene), so a one-scene batch costs a quarter
+// of the same-address operations per item.
+constexpr uint32_t kItemsPerGrab = 4;
+
+// Close a wave's run of items of scene `job`: its stats, once, and its
+// last-end stamp.  All conditions are wave-uniform (job and p.stats are).
+__device__ __forceinline__ void close_run(const BatchGroup& g,
+                                          const MarchParams* __restrict__ jobs, int job,
+                                          const RayCounts& rc) {
+  const MarchParams& p = jobs[job];
+  if (p.stats) {
+    wave_add(p.stats + ST_SAMPLES, wave_sum(rc.samples), g.sink);
+    wave_add(p.stats + ST_REEVAL, wave_sum(rc.reeval), g.sink);
+    wave_add(p.stats + ST_AUDIT_MISS, wave_sum(rc.miss), g.sink);
+    wave_add(p.stats + ST_FINE, wave_sum(rc.fine), g.sink);
+    wave_add(p.stats + ST_SKIPPED, wave_sum(rc.skipped), g.sink);
+  }
+  atomicMax(lane_slot(g.t_done + job, g.sink), (unsigned long long)wall_clock64());
+}
+
+// Every wave of a persistent grid takes items until the counter passes the
+// last one (no LDS, no barriers); march(p, v, i, j, valid, rc) renders one
+// pixel per lane, called by every lane of the wave.
+template <class March>
+__device__ __forceinline__ void batch_items(const BatchGroup& g,
+                                            const MarchParams* __restrict__ jobs, March&& march) {
+  const int lane = threadIdx.x & 63;
+  const int tile_i = 8 * g.wave_rows, tile_j = 8 * g.wave_cols;
+  for (;;) {
+    const uint32_t got =
+        atomicAdd(lane_slot(g.counter, g.sink), first_lane() ? kItemsPerGrab : 0u);
+    const uint32_t t0 = __builtin_amdgcn_readfirstlane(got);
+    if (t0 >= g.n_tiles) break;
+    const uint32_t t1 = min(t0 + kItemsPerGrab, g.n_tiles);
+    int run_job = -1;
+    RayCounts rc;
+    for (uint32_t t = t0; t < t1; ++t) {
+      // job holding item t: last job whose tile_start <= t
+      int lo = 0, hi = g.n_jobs - 1;
+      while (lo < hi) {
+        const int mid = (lo + hi + 1) >> 1;
+        if (g.tile_start[mid] <= t)
+          lo = mid;
+        else
+          hi = mid - 1;
+      }
+      const int job = __builtin_amdgcn_readfirstlane(lo);
+      if (job != run_job) {
+        if (run_job >= 0) {
+          close_run(g, jobs, run_job, rc);
+          rc = RayCounts();
+        }
+        atomicMin(lane_slot(g.t_first + job, g.sink), (unsigned long long)wall_clock64());
+        run_job = job;
+      }
+      const MarchParams& p = jobs[job];
+      const uint32_t local = t - g.tile_start[job];
+      const int tiles_i = (p.res + tile_i - 1) / tile_i, tiles_j = (p.res + tile_j - 1) / tile_j;
+      const uint32_t per_view = (uint32_t)tiles_i * (uint32_t)tiles_j;
+      const int v = (int)(local / per_view);
+      const uint32_t rem = local - (uint32_t)v * per_view;
+      const int ti = (int)(rem / (uint32_t)tiles_j), tj = (int)(rem - (uint32_t)ti * tiles_j);
+      for (int bi = 0; bi < g.wave_rows; ++bi)
+        for (int bj = 0; bj < g.wave_cols; ++bj) {
+          const int i = ti * tile_i + bi * 8 + (lane >> 3);
+          const int j = tj * tile_j + bj * 8 + (lane & 7);
+          march(p, v, i, j, i < p.res && j < p.res, rc);
+        }
+    }
+    close_run(g, jobs, run_job, rc);
+  }
+}
+
+}  // namespace xrp

@@ -14,6 +14,7 @@
 
 #include <algorithm>
 
+#include "batch_items.hpp"
 #include "line_march.hpp"
 #include "march.hpp"
 
@@ -106,6 +107,32 @@ __global__ __launch_bounds__(64) __attribute__((amdgpu_waves_per_eu(4))) void li
     if (valid) store_pixel(p, (int)v, i, j, T);
   }
   flush_counts(p.stats, rc);
+}
+
+// Batched form: the items of one group (batch.hip), every job of it with
+// line != LINE_NONE, one wave per workgroup.  10 scenes of 12-100 primitives,
+// whole call: 21.5 -> 4.5 ms (sampling march at 2 waves per SIMD before).
+template <int INTEG>
+__global__ __launch_bounds__(64) __attribute__((amdgpu_waves_per_eu(4))) void
+batch_line_kernel(BatchGroup g, const MarchParams* __restrict__ jobs) {
+  const LineSlots S = line_slots(line_lds, g.line_cap);
+  batch_items(g, jobs, [&](const MarchParams& p, int v, int i, int j, bool valid, RayCounts& rc) {
+    bool aborted;
+    const double T = line_T<INTEG, false, LINE_NONE>(p, v, i, j, valid, S, p.line_cap, rc, aborted);
+    if (valid) store_pixel(p, v, i, j, T);
+  });
+}
+
+int launch_batch_line(const BatchGroup& g, int integrator, int workgroups, void* stream) {
+  if (g.line_cap < 1) return (int)hipErrorInvalidValue;
+  const size_t lds = line_lds_bytes(g.line_cap);
+  if (integrator == INT_HIERARCHICAL)
+    hipLaunchKernelGGL((batch_line_kernel<INT_HIERARCHICAL>), dim3(workgroups), dim3(64), lds,
+                       (hipStream_t)stream, g, g.jobs);
+  else
+    hipLaunchKernelGGL((batch_line_kernel<INT_SIMPLE>), dim3(workgroups), dim3(64), lds,
+                       (hipStream_t)stream, g, g.jobs);
+  return (int)hipGetLastError();
 }
 
 template <int KIND>

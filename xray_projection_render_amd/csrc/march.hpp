@@ -237,13 +237,16 @@ struct BatchGroup {
   int32_t n_jobs;
   uint32_t n_tiles;
   int32_t wave_rows, wave_cols; // item: (8 wave_rows) x (8 wave_cols) pixels, one wave
-  int32_t pad_;
+  int32_t line_cap;             // interval march: run slots of the largest job
 };
 // Lines that take the bookkeeping atomics of a wave's lanes other than its
 // first (batch.hip lane_slot).
 constexpr int kBatchSinkBytes = 64 * 128;
 int launch_batch(const BatchGroup& g, int precision, int integrator, int workgroups,
                  void* stream);
+// The same for a group whose jobs take the interval march (line != LINE_NONE);
+// one-wave workgroups.
+int launch_batch_line(const BatchGroup& g, int integrator, int workgroups, void* stream);
 // Zero the work counters and per-job stats, and reset the timestamps,
 // with a kernel (no memset nodes, so the sequence can be graph-captured).
 int launch_batch_reset(uint32_t* counters, int n_counters, unsigned long long* t_first,
