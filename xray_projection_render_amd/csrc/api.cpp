@@ -620,7 +620,7 @@ bool line_plan(const xrp::Scene& s, const RenderJob& job, double lip, double s_e
       case K_GYROID:
         if (tess) return false;
         // path length 2 * half diagonal over the period 2 pi scale
-        if (!(6.2831853 * std::fabs(n.a) >= lip * kCubeHalfDiagonal)) return false;
+        if (!(6.2831853 * n.a >= lip * kCubeHalfDiagonal)) return false;
         ++gyroids;
         least = INFINITY;
         break;
@@ -644,12 +644,13 @@ bool line_plan(const xrp::Scene& s, const RenderJob& job, double lip, double s_e
   const size_t cap = tiles <= 1024 && !job.batched ? (size_t)kLineCapMost
                      : n_kids <= 64 ? (size_t)kLineCap
                      : n_kids <= 128 ? 2 * (size_t)kLineCap : 3 * (size_t)kLineCap;
-  mp.line_cap = tess ? (int)n_kids : (int)std::min(cap, std::max<size_t>(4, need));
+  mp.line_cap = tess ? (int)n_kids : (int)std::min(cap, need);
+  mp.line_cap = (mp.line_cap + 3) & ~3;  // whole groups (line_scan)
   // FP64 roundings of positions through the chain (64 ulps of the reach), the
   // sample table's drift, and, for cells, FP32 cell-local coordinates
   const double pos = 64.0 * 2.3e-16 * W * (1.0 + (double)s.defs.size()) + 2.0 * lip * s_err;
   mp.line_eps = (float)(pos + (tess ? 4.0 * cell / 16777216.0 : 0.0));
-  mp.line_seam = 64.0 * pos;
+  mp.line_seam = 2.0 * pos;
   return true;
 }
 
@@ -809,9 +810,8 @@ int plan_job(xrp_context* ctx, xrp_scene* sc, const RenderJob& job, LaunchPlan& 
   MarchParams line;
   std::memset(&line, 0, sizeof line);
   if (allow_line && precision == XRP_PRECISION_GUARDED && !vox_kernel &&
-      line_plan(s, job, lipschitz, table_err, line))
-    // its gyroids are evaluated at FP32 strides of the whole path
-    (void)compute_guards(s, Bw, 2.0 * kCubeHalfDiagonal, nullptr, table_err);
+      !line_plan(s, job, lipschitz, table_err, line))
+    line.line = LINE_NONE;
 
   std::vector<void*> vptr;
   if (s.has_voxels) {
@@ -1688,7 +1688,7 @@ int xrp_batch_create(xrp_context* ctx, const xrp_batch_item* items, int n_items,
       LaunchPlan pl;
       job.batched = true;
       int rc = plan_job(ctx, sc, job, pl, /*allow_voxel_kernel=*/false, /*no_alloc=*/false,
-                        /*allow_line=*/true);
+                        /*allow_line=*/!job.audit);
       if (rc) return rc;
       const Scene& s = *sc->s;
       node_off.push_back(all_nodes.size());

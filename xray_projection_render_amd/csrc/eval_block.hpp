@@ -235,8 +235,8 @@ __device__ __forceinline__ float quad_reach(float c, float b, float M, float inv
   const float q = __builtin_amdgcn_sqrtf(fmaf(b, b, 2.0f * M * c));
   return b > 0.0f ? (b + q) * inv_M : 2.0f * c * __builtin_amdgcn_rcpf(q - b);
 }
-__device__ __forceinline__ float gyroid_reach(const DevNode& n, float gg, float g1) {
-  const float th = n.f[4], band = n.g[0], M = n.g[6], e1 = n.g[7], inv_M = n.g[1];
+__device__ __forceinline__ float gyroid_reach(float gg, float g1, float th, float band, float M,
+                                              float inv_M, float e1) {
   const float ag = fabsf(gg);
   float s;
   if (ag >= th) {
@@ -246,6 +246,9 @@ __device__ __forceinline__ float gyroid_reach(const DevNode& n, float gg, float 
               quad_reach(gg + th - band, g1 - e1, M, inv_M));
   }
   return s * (1.0f - 1e-4f);
+}
+__device__ __forceinline__ float gyroid_reach(const DevNode& n, float gg, float g1) {
+  return gyroid_reach(gg, g1, n.f[4], n.g[0], n.g[6], n.g[1], n.g[7]);
 }
 
 template <int S, bool DIST>

@@ -2,14 +2,15 @@
 // of convex primitives (and wide gyroids) seen along straight object-space
 // lines.
 //
-// Bound by VALU issue: the runs of every listed child (about 70 FP32
-// instructions each) and one pass over the wave's run slots per change of
-// the density, where the sampling marches evaluated every listed child at
-// every sample they could not settle.  Whole calls, sampling march ->
-// interval march: strut lattice 30 x 500^2 6.81 -> 1.19 ms, hierarchical 12 x
-// 512^2 10.2 -> 1.46 ms; 60 primitives hierarchical 8 x 256^2 6.34 -> 0.90
-// ms; three primitives 2 x 128^2 0.100 -> 0.045 ms; 179 primitives 4 x 256^2
-// 13.2 -> 2.1 ms, hierarchical 25 -> 2.7 ms.
+// Bound by VALU issue and, on collections, by the latency of its serial
+// chains (VALU issue 38 % at 3-4 waves per SIMD): the runs of every listed
+// child (about 80 FP32 instructions each) and one pass over the wave's run
+// slots per change of the density, where the sampling marches evaluated
+// every listed child at every sample they could not settle.  Whole calls,
+// sampling march -> interval march: strut lattice 30 x 500^2 6.81 -> 1.02
+// ms, hierarchical bytes 12 x 512^2 10.2 -> 1.16 ms; 60 primitives
+// hierarchical 8 x 256^2 6.34 -> 0.52 ms; three primitives 2 x 128^2 0.100
+// -> 0.043 ms; 10 uneven scenes batched 21.5 -> 2.75 ms.
 #include <hip/hip_runtime.h>
 
 #include <algorithm>
@@ -27,6 +28,12 @@ extern __shared__ __align__(16) unsigned char line_lds[];
 template <int KIND>
 struct LineTile {
   static constexpr int I = KIND == LINE_TESS ? 32 : 8, J = 64 / I;
+};
+
+// Waves per SIMD the kernels are compiled for.
+template <int KIND>
+struct LineWaves {
+  static constexpr int n = KIND == LINE_TESS ? 4 : 3;
 };
 
 struct LinePixel {
@@ -47,37 +54,56 @@ __device__ __forceinline__ LinePixel line_pixel(const MarchParams& p) {
   return q;
 }
 
-template <int INTEG, int KIND>
-__global__ __launch_bounds__(64) __attribute__((amdgpu_waves_per_eu(4))) void line_kernel(MarchParams p) {
+// T of one pixel per lane: the march, then, ray by ray, the ones it stopped.
+// The FP64 evaluator is then called with nothing of the march live: called
+// from within it, it cost 30-50 spilled registers in the march's loops.
+template <int INTEG, bool AUDIT, int KIND>
+__device__ __forceinline__ double line_pixel_T(const MarchParams& p, int v, int i, int j,
+                                               bool valid, const LineSlots& S, int cap,
+                                               RayCounts& rc) {
+  bool stopped;
+  double T = line_T<INTEG, AUDIT, KIND>(p, v, i, j, valid, S, cap, rc, stopped);
+  for (unsigned long long m = __ballot(valid && stopped); __builtin_expect(m != 0ull, 0);
+       m &= m - 1ull) {
+    const int own = (int)__builtin_ctzll(m);
+    const double t = line_T_exact<INTEG>(p, __builtin_amdgcn_readlane(v, own),
+                                         __builtin_amdgcn_readlane(i, own),
+                                         __builtin_amdgcn_readlane(j, own), own, rc);
+    if ((int)(threadIdx.x & 63) == own) T = t;
+  }
+  return T;
+}
+
+template <int INTEG, bool AUDIT, int KIND>
+__global__ __launch_bounds__(64) __attribute__((amdgpu_waves_per_eu(LineWaves<KIND>::n))) void
+line_kernel(MarchParams p) {
   const LineSlots S = line_slots(line_lds, p.line_cap);
   const LinePixel q = line_pixel<KIND>(p);
   RayCounts rc;
-  bool aborted;
-  const double T =
-      line_T<INTEG, false, KIND>(p, q.v, q.i, q.j, q.valid, S, p.line_cap, rc, aborted);
+  const double T = line_pixel_T<INTEG, AUDIT, KIND>(p, q.v, q.i, q.j, q.valid, S, p.line_cap, rc);
   if (q.valid) store_pixel(p, q.v, q.i, q.j, T);
   flush_counts(p.stats, rc);
 }
 
-// First pass of the two-pass form: no FP64 evaluator in the kernel; rays
-// with an index that needs one are appended to p.redo_list (one atomic per
-// wave).
+// First pass of the two-pass form: the stopped rays are appended to
+// p.redo_list (one atomic per wave).
 template <int KIND>
-__global__ __launch_bounds__(64) void line_try_kernel(MarchParams p) {
+__global__ __launch_bounds__(64) __attribute__((amdgpu_waves_per_eu(LineWaves<KIND>::n))) void
+line_try_kernel(MarchParams p) {
   const LineSlots S = line_slots(line_lds, p.line_cap);
   const LinePixel q = line_pixel<KIND>(p);
   RayCounts rc;
-  bool aborted;
-  const double T =
-      line_T<INT_SIMPLE, true, KIND>(p, q.v, q.i, q.j, q.valid, S, p.line_cap, rc, aborted);
-  if (q.valid && !aborted) store_pixel(p, q.v, q.i, q.j, T);
-  const unsigned long long m = __ballot(q.valid && aborted);
+  bool stopped;
+  const double T = line_T<INT_SIMPLE, false, KIND>(p, q.v, q.i, q.j, q.valid, S, p.line_cap, rc,
+                                                   stopped);
+  if (q.valid && !stopped) store_pixel(p, q.v, q.i, q.j, T);
+  const unsigned long long m = __ballot(q.valid && stopped);
   if (m) {
     unsigned base = 0;
     if ((threadIdx.x & 63) == 0) base = atomicAdd(p.counts, (unsigned)__popcll(m));
     base = (unsigned)__shfl((int)base, 0, 64);
     const unsigned e = base + (unsigned)__popcll(m & __lanemask_lt());
-    if (q.valid && aborted) {
+    if (q.valid && stopped) {
       if (e < p.redo_cap)
         p.redo_list[e] = ((unsigned)q.v * (unsigned)p.res + (unsigned)q.i) * (unsigned)p.res +
                          (unsigned)q.j;
@@ -88,37 +114,28 @@ __global__ __launch_bounds__(64) void line_try_kernel(MarchParams p) {
   flush_counts(p.stats, rc);
 }
 
-// Second pass: the listed rays, 64 per wave in list order (grid-stride).
-template <int KIND>
-__global__ __launch_bounds__(64) __attribute__((amdgpu_waves_per_eu(4))) void line_redo_kernel(MarchParams p) {
-  const LineSlots S = line_slots(line_lds, p.line_cap);
+// Second pass: one listed ray per wave (grid-stride).
+__global__ __launch_bounds__(64) void line_redo_kernel(MarchParams p) {
   const unsigned n = min(p.counts[0], p.redo_cap);
   const unsigned rr = (unsigned)p.res * (unsigned)p.res;
   RayCounts rc;
-  for (unsigned base = blockIdx.x * 64u; base < n; base += gridDim.x * 64u) {
-    const unsigned e = base + threadIdx.x;
-    const bool valid = e < n;
-    const unsigned id = valid ? p.redo_list[e] : 0u;
-    const unsigned v = id / rr, pix = id - v * rr;
+  for (unsigned e = blockIdx.x; e < n; e += gridDim.x) {
+    const unsigned id = p.redo_list[e], v = id / rr, pix = id - v * rr;
     const int i = (int)(pix / (unsigned)p.res), j = (int)(pix - (unsigned)i * p.res);
-    bool aborted;
-    const double T =
-        line_T<INT_SIMPLE, false, KIND>(p, (int)v, i, j, valid, S, p.line_cap, rc, aborted);
-    if (valid) store_pixel(p, (int)v, i, j, T);
+    const double T = line_T_exact<INT_SIMPLE>(p, (int)v, i, j, 0, rc);
+    if (threadIdx.x == 0) store_pixel(p, (int)v, i, j, T);
   }
   flush_counts(p.stats, rc);
 }
 
 // Batched form: the items of one group (batch.hip), every job of it with
-// line != LINE_NONE, one wave per workgroup.  10 scenes of 12-100 primitives,
-// whole call: 21.5 -> 4.5 ms (sampling march at 2 waves per SIMD before).
+// line != LINE_NONE, one wave per workgroup.
 template <int INTEG>
 __global__ __launch_bounds__(64) __attribute__((amdgpu_waves_per_eu(4))) void
 batch_line_kernel(BatchGroup g, const MarchParams* __restrict__ jobs) {
   const LineSlots S = line_slots(line_lds, g.line_cap);
   batch_items(g, jobs, [&](const MarchParams& p, int v, int i, int j, bool valid, RayCounts& rc) {
-    bool aborted;
-    const double T = line_T<INTEG, false, LINE_NONE>(p, v, i, j, valid, S, p.line_cap, rc, aborted);
+    const double T = line_pixel_T<INTEG, false, LINE_NONE>(p, v, i, j, valid, S, p.line_cap, rc);
     if (valid) store_pixel(p, v, i, j, T);
   });
 }
@@ -141,14 +158,17 @@ static int launch_kind(const MarchParams& p, int integrator, hipStream_t s) {
   const dim3 block(64);
   const dim3 grid(((p.res + TI - 1) / TI) * ((p.res + TJ - 1) / TJ), p.n_views);
   const size_t lds = line_lds_bytes(p.line_cap);
-  if (integrator == INT_HIERARCHICAL) {
-    hipLaunchKernelGGL((line_kernel<INT_HIERARCHICAL, KIND>), grid, block, lds, s, p);
-  } else if (p.redo_list && !p.audit) {
-    const dim3 grid2(std::min((p.redo_cap + 63u) / 64u, 4096u));
+  if (integrator == INT_HIERARCHICAL && p.audit) {
+    hipLaunchKernelGGL((line_kernel<INT_HIERARCHICAL, true, KIND>), grid, block, lds, s, p);
+  } else if (integrator == INT_HIERARCHICAL) {
+    hipLaunchKernelGGL((line_kernel<INT_HIERARCHICAL, false, KIND>), grid, block, lds, s, p);
+  } else if (p.audit) {
+    hipLaunchKernelGGL((line_kernel<INT_SIMPLE, true, KIND>), grid, block, lds, s, p);
+  } else if (p.redo_list) {
     hipLaunchKernelGGL((line_try_kernel<KIND>), grid, block, lds, s, p);
-    hipLaunchKernelGGL((line_redo_kernel<KIND>), grid2, block, lds, s, p);
+    hipLaunchKernelGGL(line_redo_kernel, dim3(std::min(p.redo_cap, 4096u)), block, 0, s, p);
   } else {
-    hipLaunchKernelGGL((line_kernel<INT_SIMPLE, KIND>), grid, block, lds, s, p);
+    hipLaunchKernelGGL((line_kernel<INT_SIMPLE, false, KIND>), grid, block, lds, s, p);
   }
   return (int)hipGetLastError();
 }
