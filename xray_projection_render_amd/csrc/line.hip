@@ -129,9 +129,11 @@ __global__ __launch_bounds__(64) void line_redo_kernel(MarchParams p) {
 }
 
 // Batched form: the items of one group (batch.hip), every job of it with
-// line != LINE_NONE, one wave per workgroup.
+// line != LINE_NONE, one wave per workgroup.  2 waves per SIMD: the item loop
+// spills at 3, with the same time (10 scenes 2.70 against 2.69 ms; the run
+// slots' LDS admits 2 to 4).
 template <int INTEG>
-__global__ __launch_bounds__(64) __attribute__((amdgpu_waves_per_eu(4))) void
+__global__ __launch_bounds__(64) __attribute__((amdgpu_waves_per_eu(2))) void
 batch_line_kernel(BatchGroup g, const MarchParams* __restrict__ jobs) {
   const LineSlots S = line_slots(line_lds, g.line_cap);
   batch_items(g, jobs, [&](const MarchParams& p, int v, int i, int j, bool valid, RayCounts& rc) {

@@ -324,13 +324,10 @@ __device__ __forceinline__ LineSpan<F> line_span(const Node& n, F w0, F w1, F w2
   return q;
 }
 
-// The FP64 evaluators are called (rarely) out of line: inlined, they set the
-// register budget of the whole march (200-240 VGPRs, 2 waves per SIMD).
-// Their pointers and node index are the same on every lane.  In a function
-// the compiler cannot tell, and reads the node records with vector loads,
-// one memory latency per field (a 36-strut cell: 0.33 ms per call, most of
-// the kernel where a column of rays lies in a cell face); through the
-// constant address space they come as scalar loads.
+// The full FP64 evaluator, for the rays that ties stop.  The node records
+// come through the constant address space: read through plain pointers in a
+// called function they were vector loads, one memory latency per field (a
+// 36-strut cell: 0.33 ms per call).
 typedef const DevNode __attribute__((address_space(4))) * LineNodes;
 typedef const DevDeform __attribute__((address_space(4))) * LineDefs;
 __device__ __forceinline__ unsigned long long line_uniform(const void* p) {
@@ -382,7 +379,7 @@ __device__ __forceinline__ bool line_wrap64(LineNodes N, double& X, double& Y, d
   return !(X < b[6] || X > b[9] || Y < b[7] || Y > b[10] || Z < b[8] || Z > b[11]);
 }
 // Density of the whole tree (one of line_plan's forms) at a world point.
-__device__ __noinline__ double line_density64(const DevNode* nodes, const DevDeform* defs,
+__device__ __forceinline__ double line_density64(const DevNode* nodes, const DevDeform* defs,
                                               int n_defs, double x, double y, double z) {
   const LineNodes N = (LineNodes)line_uniform(nodes);
   line_deform64((LineDefs)line_uniform(defs), __builtin_amdgcn_readfirstlane(n_defs), x, y, z);
