@@ -133,8 +133,8 @@ struct xrp_context {
   double table_smin = NAN, table_smax = NAN, table_ds = NAN;
   std::vector<double> table_host;
   std::set<xrp_scene*> scenes;  // scenes holding device copies here
-  // xrp_render_volume_projections: the last volume as a scene, reused while
-  // the caller passes the same grid
+  // xrp_render_volume_projections: a scene of the last volume's dimensions,
+  // whose device buffers (and no host copy) are kept between calls
   xrp_scene* vol_scene = nullptr;
   // the fixed scratch region of xrp_render_device_noalloc on this device
   void* scratch = nullptr;
@@ -464,50 +464,6 @@ bool cull_enabled() {
   return on;
 }
 
-// [z][x][y] grid -> 4x4x4 bricks ordered (bz, bx, by), voxels (lz, lx, ly)
-// inside a brick; padding voxels are zero and never read.
-std::vector<float> brick4(const std::vector<float>& v, int nx, int ny, int nz) {
-  int bx = (nx + 3) / 4, by = (ny + 3) / 4, bz = (nz + 3) / 4;
-  std::vector<float> out((size_t)bx * by * bz * 64, 0.0f);
-  for (int z = 0; z < nz; ++z)
-    for (int x = 0; x < nx; ++x)
-      for (int y = 0; y < ny; ++y) {
-        size_t b = ((size_t)(z >> 2) * bx + (x >> 2)) * by + (y >> 2);
-        size_t l = (size_t)(z & 3) * 16 + (x & 3) * 4 + (y & 3);
-        out[b * 64 + l] = v[((size_t)z * nx + x) * ny + y];
-      }
-  return out;
-}
-
-// Brick-order copies with each voxel's upper-y neighbour (PAIR: v[y], v[y1])
-// or upper-y and upper-z neighbours (QUAD: v[z][y], v[z1][y], v[z][y1],
-// v[z1][y1]) stored beside it, upper indices clamped to N-1 as
-// objects.go:811-830 clamps them, so a cell's 8 corners come in 4 or 2 wide
-// loads.
-std::vector<float> brick4_wide(const std::vector<float>& v, int nx, int ny, int nz, int w) {
-  int bx = (nx + 3) / 4, by = (ny + 3) / 4, bz = (nz + 3) / 4;
-  std::vector<float> out((size_t)bx * by * bz * 64 * w, 0.0f);
-  auto at = [&](int z, int x, int y) { return v[((size_t)z * nx + x) * ny + y]; };
-  for (int z = 0; z < nz; ++z)
-    for (int x = 0; x < nx; ++x)
-      for (int y = 0; y < ny; ++y) {
-        size_t b = ((size_t)(z >> 2) * bx + (x >> 2)) * by + (y >> 2);
-        size_t l = (size_t)(z & 3) * 16 + (x & 3) * 4 + (y & 3);
-        float* o = &out[(b * 64 + l) * w];
-        const int y1 = std::min(y + 1, ny - 1), z1 = std::min(z + 1, nz - 1);
-        if (w == 2) {
-          o[0] = at(z, x, y);
-          o[1] = at(z, x, y1);
-        } else {
-          o[0] = at(z, x, y);
-          o[1] = at(z1, x, y);
-          o[2] = at(z, x, y1);
-          o[3] = at(z1, x, y1);
-        }
-      }
-  return out;
-}
-
 // World -> object map of a chain of affine/linear/rigid deformations.
 bool compose_linear(const std::vector<xrp::HDeform>& defs, double M[9], double t[3]) {
   double m[9] = {1, 0, 0, 0, 1, 0, 0, 0, 1}, v[3] = {0, 0, 0};
@@ -657,11 +613,19 @@ bool line_plan(const xrp::Scene& s, const RenderJob& job, double lip, double s_e
 // Brick-order copies of a voxel root that the voxel-root kernel reads.
 enum BrickSlot { SLOT_PLAIN = 0, SLOT_PAIR = 1, SLOT_QUAD = 2, N_SLOTS = 3 };
 
+size_t mp_bricks(const xrp::HNode& n) {
+  return (size_t)((n.nx + 3) / 4) * ((n.ny + 3) / 4) * ((n.nz + 3) / 4);
+}
+int slot_width(int slot) { return slot == SLOT_PLAIN ? 1 : slot == SLOT_PAIR ? 2 : 4; }
+size_t brick_bytes(const xrp::HNode& n, int slot) {
+  return mp_bricks(n) * 64 * sizeof(float) * slot_width(slot);
+}
+
 // Device copies of a scene's voxel grids on one context: the linear copy of
 // every voxel node (preorder, matching the flattened node order), then, for
-// a voxel root, N_SLOTS brick-copy slots.  A brick slot is filled on first
-// use (slot < 0 asks for none), so a scene holds only the copies its
-// layouts need.
+// a voxel root, N_SLOTS brick-copy slots.  A brick slot is built from the
+// linear copy, on the device, on first use (slot < 0 asks for none), so a
+// scene holds only the copies its layouts need.
 int upload_voxels(xrp_context* ctx, xrp_scene* sc, std::vector<void*>& ptrs,
                   int slot = -1, bool no_alloc = false) {
   std::lock_guard<std::mutex> g(g_registry_mu);
@@ -669,10 +633,13 @@ int upload_voxels(xrp_context* ctx, xrp_scene* sc, std::vector<void*>& ptrs,
       "voxel grid not resident on this context: render the scene once with "
       "xrp_render or xrp_render_device first (this call allocates nothing)";
   const bool root_vox = sc->s->root.kind == xrp::K_VOXEL;
-  auto put = [](const std::vector<float>& host, size_t bytes, void*& p) -> hipError_t {
+  // on the context's stream, which reads the copies
+  auto put = [ctx](const std::vector<float>& host, size_t bytes, void*& p) -> hipError_t {
     p = nullptr;
     hipError_t e = hipMalloc(&p, std::max<size_t>(bytes, 4));
-    if (e == hipSuccess) e = hipMemcpy(p, host.data(), bytes, hipMemcpyHostToDevice);
+    if (e == hipSuccess)
+      e = hipMemcpyAsync(p, host.data(), bytes, hipMemcpyHostToDevice, ctx->stream);
+    if (e == hipSuccess) e = hipStreamSynchronize(ctx->stream);
     if (e != hipSuccess && p) {
       (void)hipFree(p);
       p = nullptr;
@@ -709,24 +676,50 @@ int upload_voxels(xrp_context* ctx, xrp_scene* sc, std::vector<void*>& ptrs,
     if (!p && no_alloc) return fail(XRP_ERR_UNSUPPORTED, not_resident);
     if (!p) {
       const xrp::HNode& n = sc->s->root;
-      std::vector<float> br;
-      if (slot == SLOT_PLAIN) {
-        br = brick4(*n.vox, n.nx, n.ny, n.nz);
-      } else {
-        br = brick4_wide(*n.vox, n.nx, n.ny, n.nz, slot == SLOT_PAIR ? 2 : 4);
-      }
-      hipError_t e = put(br, br.size() * sizeof(float), p);
-      if (e != hipSuccess)
+      hipError_t e = hipMalloc(&p, brick_bytes(n, slot));
+      if (e == hipSuccess)
+        e = (hipError_t)xrp::launch_bricks((const float*)out[0], n.nx, n.ny, n.nz,
+                                           slot_width(slot), (float*)p, ctx->stream);
+      if (e != hipSuccess) {
+        if (p) (void)hipFree(p);
+        p = nullptr;
         return fail(XRP_ERR_ALLOC, std::string("voxel upload failed: ") +
                                        hipGetErrorString(e));
+      }
     }
   }
   ptrs = out;
   return XRP_OK;
 }
 
-size_t mp_bricks(const xrp::HNode& n) {
-  return (size_t)((n.nx + 3) / 4) * ((n.ny + 3) / 4) * ((n.nz + 3) / 4);
+// Copies new values into a voxel root's device grid (allocated on first use)
+// and builds the brick copies held for it again.
+int refresh_volume(xrp_context* ctx, xrp_scene* sc, const float* volume) {
+  std::lock_guard<std::mutex> g(g_registry_mu);
+  const xrp::HNode& n = sc->s->root;
+  const size_t bytes = (size_t)n.nx * n.ny * n.nz * sizeof(float);
+  auto it = sc->uploads.find(ctx);
+  if (it == sc->uploads.end()) {
+    void* p = nullptr;
+    hipError_t e = hipMalloc(&p, bytes);
+    if (e != hipSuccess)
+      return fail(XRP_ERR_ALLOC, std::string("voxel upload failed: ") + hipGetErrorString(e));
+    std::vector<void*> out(1, p);
+    out.insert(out.end(), N_SLOTS, nullptr);
+    it = sc->uploads.emplace(ctx, std::move(out)).first;
+    ctx->scenes.insert(sc);
+  }
+  const std::vector<void*>& out = it->second;
+  HIPCHK(hipMemcpyAsync(out[0], volume, bytes, hipMemcpyHostToDevice, ctx->stream));
+  for (int slot = 0; slot < N_SLOTS; ++slot)
+    if (void* p = out[out.size() - N_SLOTS + slot]) {
+      int e = xrp::launch_bricks((const float*)out[0], n.nx, n.ny, n.nz, slot_width(slot),
+                                 (float*)p, ctx->stream);
+      if (e) return fail(XRP_ERR_DEVICE, hipGetErrorString((hipError_t)e));
+    }
+  // the caller's memory is read until the copy is done
+  HIPCHK(hipStreamSynchronize(ctx->stream));
+  return XRP_OK;
 }
 
 // Everything a launch of one scene needs, computed on the host: the
@@ -1389,22 +1382,25 @@ int xrp_render_volume_projections(xrp_context* ctx, const float* volume, int nx,
     }
     std::lock_guard<std::mutex> g(ctx->mu);
     HIPCHK(hipSetDevice(ctx->device));
-    // The volume's scene, with its device copy and brick copies, stays on
-    // the context while the caller passes the same dimensions and values.
-    const size_t nvox = (size_t)nx * ny * nz;
+    // The volume's scene, with its device buffers, stays on the context for
+    // calls with the same dimensions; the values are copied over on every
+    // call and the brick copies built from them again there (comparing the
+    // volume with a host copy of the last one costs more than the copy over).
     xrp_scene*& sc = ctx->vol_scene;
     if (sc) {
       const xrp::HNode& r = sc->s->root;
-      if (r.nx != nx || r.ny != ny || r.nz != nz ||
-          std::memcmp(r.vox->data(), volume, nvox * sizeof(float)) != 0) {
+      if (r.nx != nx || r.ny != ny || r.nz != nz) {
         xrp_scene_destroy(sc);
         sc = nullptr;
       }
     }
     if (!sc) {
-      int rc = xrp_scene_create_voxels(volume, nx, ny, nz, nullptr, XRP_NUMBERS_JSON, &sc);
-      if (rc) return rc;
+      std::unique_ptr<xrp_scene> made(new xrp_scene());
+      made->s = xrp::voxel_scene(nullptr, nx, ny, nz, nullptr, xrp::NUMBERS_JSON);
+      sc = made.release();
     }
+    int rc = refresh_volume(ctx, sc, volume);
+    if (rc) return rc;
     const size_t img = (size_t)image_res * image_res;
     HIPCHK(ctx->out.ensure(img * n_cams * sizeof(float)));
     // Consecutive cameras sharing (fov, R) go into one launch.

@@ -204,6 +204,10 @@ inline bool voxel_layout_linear(int layout) {
   return layout == VOX_LINEAR || layout == VOX_LINEAR_CACHED;
 }
 int launch_voxel(const MarchParams& p, int layout, void* stream);
+// Brick copy of a device [z][x][y] grid (width 1, 2 or 4 floats an element;
+// under 2^32 elements).
+int launch_bricks(const float* grid, int nx, int ny, int nz, int width, float* out,
+                  void* stream);
 // L2 read-bandwidth probe: workgroups x 256 lanes each read iters 16-byte
 // words from a buffer of l2_probe_buffer_bytes(); out gets workgroups x 256
 // words.

@@ -1037,8 +1037,8 @@ std::unique_ptr<Scene> voxel_scene(const float* rho, int nx, int ny, int nz,
   s->root.nx = nx;
   s->root.ny = ny;
   s->root.nz = nz;
-  s->root.vox = std::make_shared<std::vector<float>>(
-      rho, rho + (size_t)nx * ny * nz);
+  s->root.vox = rho ? std::make_shared<std::vector<float>>(rho, rho + (size_t)nx * ny * nz)
+                    : std::make_shared<std::vector<float>>();
   if (deformation && !deformation->is_null())
     parse_deformation(*deformation, Num{numbers == NUMBERS_JSON}, s->defs, 0);
   finalize_scene(*s);

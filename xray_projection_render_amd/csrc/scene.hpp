@@ -73,7 +73,8 @@ std::unique_ptr<Scene> load_scene(const json::Value& object,
                                   const json::Value* deformation,
                                   NumberMode numbers,
                                   const std::string& base_dir);
-// Voxel grid scene from caller memory ([z][x][y], float32 densities).
+// Voxel grid scene from caller memory ([z][x][y], float32 densities); rho
+// NULL: the dimensions alone, without host values.
 std::unique_ptr<Scene> voxel_scene(const float* rho, int nx, int ny, int nz,
                                    const json::Value* deformation,
                                    NumberMode numbers);
