@@ -32,6 +32,7 @@ DEVICE = ["-x", "hip", "--offload-arch=" + ARCH,
 SOURCES = [
     ("march.hip", True),
     ("line.hip", True),
+    ("gyroid.hip", True),
     ("voxel.hip", True),
     ("batch.hip", True),
     ("surrogate.hip", True),

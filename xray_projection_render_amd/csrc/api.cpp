@@ -132,6 +132,7 @@ struct xrp_context {
   int table_mode = -1;
   double table_smin = NAN, table_smax = NAN, table_ds = NAN;
   std::vector<double> table_host;
+  int table_fine_most = 0;  // hierarchical: most fine samples of a step (15: 15 or more)
   std::set<xrp_scene*> scenes;  // scenes holding device copies here
   // xrp_render_volume_projections: a scene of the last volume's dimensions,
   // whose device buffers (and no host copy) are kept between calls
@@ -722,6 +723,55 @@ int refresh_volume(xrp_context* ctx, xrp_scene* sc, const float* volume) {
   return XRP_OK;
 }
 
+// The gyroid march (gyroid_march.hpp) takes a guarded render whose root is a
+// seamless tessellation of one gyroid and whose march uses the second-order
+// reach: returns the gyroid's node, with mp.gyro_rho, or 0.  The phase is
+// taken without the wrap, so the cells' sides may differ from whole periods
+// by no more, over all of the box, than the FP32 rounding of a coordinate.
+//
+// mp.gyro_band, the error bound of the march's FP32 g (u = 2^-24): a
+// coordinate is off by delta from the position, u (bounds + |centre|) from
+// the subtraction of the centre and u bounds from the cells' sides; the
+// phase, reduced by one fma, by pi u twice.  |grad g| <= 1.77 (compute_guards)
+// over three coordinates so off: 1.77 sqrt(3) < 3.07 times that; the hardware
+// sine and cosine enter three products of two; 16 u for the products, the
+// sums and the level.  5 % in hand for the second-order terms with the
+// hierarchical integrator, whose fine samples lie at surfaces (a twelfth of
+// the general march's band: check and redo passes of 24 x 1024^2 rays 4.0 ->
+// 1.6 ms); four times the bound, as in compute_guards, with the simple one,
+// which has few samples in the band (resolve pass of 16 x 512^2: 36 us).
+int gyroid_plan(const xrp::Scene& s, const std::vector<xrp::DevNode>& nodes, double delta,
+                bool simple, xrp::MarchParams& mp) {
+  using namespace xrp;
+  const char* e = std::getenv("XRP_GYROID");
+  if (e && std::strcmp(e, "0") == 0) return 0;
+  if (!mp.vel || !mp.clip || nodes.size() != 3 || nodes[0].kind != K_TESS ||
+      nodes[0].g[2] == 0.0f || nodes[1].kind != K_COLL || nodes[2].kind != K_GYROID)
+    return 0;
+  const DevNode &t = nodes[0], &g = nodes[2];
+  if (!(g.d[3] > 0.0) || !std::isfinite(g.d[4])) return 0;
+  const double period = 2.0 * M_PI * g.d[3];
+  double bb = 0.0;
+  for (int k = 0; k < 6; ++k) bb = std::max(bb, std::fabs(t.d[k]));
+  for (int a = 0; a < 3; ++a) {
+    const double side = t.d[9 + a] - t.d[6 + a];
+    const double off = std::fabs(side - std::round(side / period) * period);
+    const double cells = (bb + std::fabs(t.d[6 + a])) / side + 1.0;
+    if (!(cells * off <= bb / 16777216.0) || !(cells < 1e6)) return 0;
+  }
+  double cm = 0.0;
+  for (int k = 0; k < 3; ++k) cm = std::max(cm, std::fabs(g.d[k]));
+  const double u = 1.0 / 16777216.0;
+  const double eq = (delta + u * (2.0 * bb + cm)) / g.d[3] + 2.0 * M_PI * u;
+  const double kappa = simple ? 4.0 : 1.05;
+  mp.gyro_band = (float)(kappa * (3.07 * eq + 6.0 * kHwSinCosErr + 16.0 * u));
+  mp.gyro_tanh = s.ddefs.size() == 1 && s.ddefs[0].kind == D_TANH ? 1 : 0;
+  const double rho = g.d[5];
+  mp.gyro_rho = nodes[1].greedy && rho > 0.0 ? rho : rho < 0.0 ? 0.0 : rho > 1.0 ? 1.0 : rho;
+  const double rr = mp.gyro_rho * mp.dm;
+  return std::isfinite(rr) && rr != 0.0 ? 2 : 0;
+}
+
 // Everything a launch of one scene needs, computed on the host: the
 // resolved precision, the sample table, the node table with guard bands and
 // voxel pointers, and the launch parameters.  Device pointers for nodes,
@@ -788,10 +838,11 @@ int plan_job(xrp_context* ctx, xrp_scene* sc, const RenderJob& job, LaunchPlan& 
     double step = job.integrator == XRP_INTEGRATE_SIMPLE ? 32.0 * job.ds : 0.0;
     table_err = (10.0 * K + 4.0) * 2.3e-16 * std::max(std::fabs(smin), std::fabs(smax));
     // simple march anchors: smin + k ds against the table's K accumulated
-    // additions (each off by at most half an ulp of |s|)
+    // additions (each off by at most half an ulp of |s|); the hierarchical
+    // gyroid march's positions the same, on the fine grid
     double s_err = job.integrator == XRP_INTEGRATE_SIMPLE
                        ? (K + 4.0) * 2.3e-16 * std::max(std::fabs(smin), std::fabs(smax))
-                       : 0.0;
+                       : table_err;
     delta = compute_guards(s, Bw, step, &lipschitz, s_err);
     // The bands keep the result exact at any delta; they only cost time when
     // wide.  Fall back to FP64 when the FP32 position error reaches a tenth
@@ -851,6 +902,7 @@ int plan_job(xrp_context* ctx, xrp_scene* sc, const RenderJob& job, LaunchPlan& 
       for (const auto& n : pl.nodes)
         if (n.kind == K_GYROID && n.g[6] > 0.0f) mp.vel = 1;
   }
+  mp.gyro = gyroid_plan(s, pl.nodes, delta, job.integrator == XRP_INTEGRATE_SIMPLE, mp);
   // Samples per node visit of the per-scene guarded simple march: with the
   // safe radius, 2 is faster on small trees (lattice cell 10 nodes: 6 %
   // faster than 1), 4 on large collections, whose node walk it amortises
@@ -867,6 +919,7 @@ int plan_job(xrp_context* ctx, xrp_scene* sc, const RenderJob& job, LaunchPlan& 
     mp.queue = std::strcmp(e, "1") == 0 ? 1 : 0;
   if (const char* e = std::getenv("XRP_TILE"))  // for comparison: 32x2 or 2x32
     mp.tile_j32 = std::strcmp(e, "2x32") == 0 ? 1 : 0;
+  if (mp.block != 1 || mp.queue || mp.tile_j32) mp.gyro = 0;
   // Per-wave culling of the root collection's children (guarded marches):
   // needs the deformations composed to one affine map, so that rays stay
   // lines in object space.  From 8 children up: on the 3-child CSG scene
@@ -1013,11 +1066,27 @@ int render_core(xrp_context* ctx, xrp_scene* sc, const RenderJob& job,
     vpc = std::max(1, std::min(vpc, std::atoi(e)));
   const int n_chunks = (nv + vpc - 1) / vpc;
 
-  // Sample table (device copy cached per context).
+  // Sample table (device copy cached per context); after the coarse samples,
+  // the number of fine samples of each coarse step (main.go:180-186).
   const double smin = job.R - kCubeHalfDiagonal, smax = job.R + kCubeHalfDiagonal;
   if (!fixed && (ctx->table_mode != job.integrator || ctx->table_smin != smin ||
                  ctx->table_smax != smax || ctx->table_ds != job.ds)) {
+    const size_t K = pl.table.size();
+    ctx->table_mode = -1;
     ctx->table_host = pl.table;
+    ctx->table_host.resize(hier ? K + (K + 7) / 8 : K);
+    ctx->table_fine_most = 0;
+    if (hier) {
+      uint8_t* fine = (uint8_t*)(ctx->table_host.data() + K);
+      for (size_t n = 0; n < K; ++n) {
+        int m = 0;
+        for (double left = (n ? pl.table[n - 1] : smin) + job.ds / 10.0;
+             left < pl.table[n] && m < 15; left += job.ds / 10.0)
+          ++m;
+        fine[n] = (uint8_t)m;
+        ctx->table_fine_most = std::max(ctx->table_fine_most, m);
+      }
+    }
     HIPCHK(ctx->table.ensure(std::max<size_t>(1, ctx->table_host.size()) *
                              sizeof(double)));
     if (!ctx->table_host.empty())
@@ -1096,6 +1165,8 @@ int render_core(xrp_context* ctx, xrp_scene* sc, const RenderJob& job,
   mp.views = (const DevView*)(db + o_views);
   mp.s_table = fixed ? (const double*)(db + o_table) : (const double*)ctx->table.p;
   mp.stats = (unsigned long long*)(db + o_stats);
+  if (fixed || (hier && ctx->table_fine_most > 14)) mp.gyro = 0;
+  if (mp.gyro && hier) mp.fine_n = (const uint8_t*)(mp.s_table + pl.table.size());
   (void)res;
 
   HIPCHK(hipEventRecord(ctx->ev0, ctx->stream));
@@ -1131,6 +1202,7 @@ int render_core(xrp_context* ctx, xrp_scene* sc, const RenderJob& job,
                                                              : INT_SIMPLE;
     int e = vox_kernel ? launch_voxel(mp, layout, ctx->stream)
             : line     ? launch_line(mp, integ, ctx->stream)
+            : mp.gyro  ? launch_gyroid(mp, integ, ctx->stream)
                        : launch_march(mp, prec, integ, ctx->stream);
     if (e != 0) {
       // the staging copy may still be reading the pinned buffer

@@ -79,7 +79,8 @@ static_assert(sizeof(DevNode) == 256, "DevNode must stay 256 bytes");
 //  BOX    f: cx cy cz hx hy hz rho  d: cx cy cz hx hy hz rho    (h = 0.5*side)
 //  PPED   f: ox oy oz m00..m22 rho  d: ox oy oz m[9] rho  (m = M^-1 column-major)
 //  CYL    f: p0(3) v(3) vv inv_vv r2 rho   d: p0(3) v(3) vv r rho
-//  GYROID f: cx cy cz inv_scale thick rho inv_scale/(2 pi)
+//  GYROID f: cx cy cz inv_scale thick rho inv_scale/(2 pi), and what its
+//         rounding lost
 //         d: cx cy cz scale thick rho
 //  TESS   f: bounds(6) ucmin(3) dx dy dz inv_dx inv_dy inv_dz
 //         d: bounds(6) ucmin(3) ucmax(3)   (dx = ucmax - ucmin, objects.go:574)

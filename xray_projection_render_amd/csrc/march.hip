@@ -24,6 +24,7 @@
 #include "eval_device.hpp"
 #include "march.hpp"
 #include "march_ray.hpp"
+#include "two_pass.hpp"
 
 namespace xrp {
 
@@ -66,84 +67,6 @@ march_kernel(MarchParams p) {
   RayCounts rc;
   march_ray<PREC, INTEG, 1, B, PREC == PREC_GUARDED && INTEG == INT_SIMPLE && (B == 4 || Q)>(
       p, blockIdx.y, i, j, i < p.res && j < p.res, rc);
-  flush_counts(p.stats, rc);
-}
-
-// End of a first-pass wave of the two-pass marches; every lane calls it.
-// A ray with nothing deferred stores its pixel (SPEC: every ray not stopped
-// does, its listed samples to be checked, and its counts follow its items
-// in defer_k: samples, fine samples, settled samples).  The rays with
-// deferred items are appended, with T and the items (ts.ks), to the
-// resolve pass's lists in lane order (an exclusive scan of the counts over
-// the wave, one atomic per wave and list).  The stopped ones, and a wave's deferring rays when
-// the lists are full, go to p.redo_list.  The counts of a ray go to rc only
-// when it is not marched again.
-template <bool SPEC = false>
-__device__ __forceinline__ void try_finish(const MarchParams& p, int v, int i, int j,
-                                           bool valid, double T, TryState& ts,
-                                           RayCounts& rc) {
-  const int lane = threadIdx.x & 63;
-  const unsigned id = ((unsigned)v * (unsigned)p.res + (unsigned)i) * (unsigned)p.res +
-                      (unsigned)j;
-  if (valid && !ts.aborted && (SPEC || ts.cnt == 0)) store_pixel(p, v, i, j, T);
-  bool defer = valid && !ts.aborted && ts.cnt > 0;
-  const unsigned kc = ts.cnt + (SPEC ? 3u : 0u);  // words in defer_k
-  const unsigned long long dm = __ballot(defer);
-  if (dm) {
-    unsigned incl = defer ? kc : 0u;
-#pragma unroll
-    for (int off = 1; off < 64; off <<= 1) {
-      const unsigned t = (unsigned)__shfl_up((int)incl, off, 64);
-      if (lane >= off) incl += t;
-    }
-    const unsigned total = (unsigned)__shfl((int)incl, 63, 64);
-    unsigned eb = 0, kb = 0;
-    if (lane == 0) {
-      eb = atomicAdd(p.counts + 1, (unsigned)__popcll(dm));
-      kb = atomicAdd(p.counts + 2, total);
-    }
-    eb = (unsigned)__shfl((int)eb, 0, 64);
-    kb = (unsigned)__shfl((int)kb, 0, 64);
-    const bool fits = eb + (unsigned)__popcll(dm) <= p.defer_cap && kb + total <= p.k_cap;
-    if (defer && fits) {
-      const unsigned e = eb + (unsigned)__popcll(dm & __lanemask_lt());
-      const unsigned k0 = kb + incl - kc;
-      p.defer_T[e] = T;
-      p.defer_ray[e] = id;
-      p.defer_cnt[e] = ts.cnt;
-      p.defer_kfirst[e] = k0;
-      for (unsigned c = 0; c < ts.cnt; ++c) p.defer_k[k0 + c] = ts.ks[c];
-      if (SPEC) {
-        p.defer_k[k0 + ts.cnt] = ts.samples;
-        p.defer_k[k0 + ts.cnt + 1] = ts.fine;
-        p.defer_k[k0 + ts.cnt + 2] = ts.skipped;
-      }
-    } else if (defer) {
-      // the lists are full: the wave's rays go to the redo list, and its
-      // entries below the cap are marked empty for the resolve pass
-      const unsigned e = eb + (unsigned)__popcll(dm & __lanemask_lt());
-      if (e < p.defer_cap) p.defer_cnt[e] = 0u;
-      ts.aborted = true;
-    }
-  }
-  if (valid && !ts.aborted) {
-    rc.samples += ts.samples;
-    rc.skipped += ts.skipped;
-    rc.fine += ts.fine;
-  }
-  const unsigned long long m = __ballot(valid && ts.aborted);
-  if (m) {
-    unsigned base = 0;
-    if (lane == 0) base = atomicAdd(p.counts, (unsigned)__popcll(m));
-    base = (unsigned)__shfl((int)base, 0, 64);
-    const unsigned e = base + (unsigned)__popcll(m & __lanemask_lt());
-    if (valid && ts.aborted) {
-      if (e < p.redo_cap)
-        p.redo_list[e] = id;
-      else
-        p.counts[3] = 1u;  // no room: the caller renders again in one pass
-    }
-  }
   flush_counts(p.stats, rc);
 }
 
@@ -277,7 +200,8 @@ march_hier_check_kernel(MarchParams p) {
       }
       bool wrong = false;
       if (has) {
-        const unsigned item = p.defer_k[ko + c], nn = item >> 4, m = item & 15u;
+        const unsigned item = p.defer_k[ko + c], nn = (item & 0x7fffffffu) >> 4,
+                       m = item & 15u;
         double sq[1];
         if (m == 15u) {
           sq[0] = p.s_table[nn];
@@ -285,11 +209,13 @@ march_hier_check_kernel(MarchParams p) {
           sq[0] = (nn == 0 ? p.smin : p.s_table[nn - 1]) + dsf;
           for (unsigned q = 0; q < m; ++q) sq[0] += dsf;
         }
-        double f32[1];
+        // the gyroid march lists the membership it used in bit 31
+        double f32[1] = {(item >> 31) ? p.gyro_rho : 0.0};
         unsigned amb;
         unsigned long long unused = 0;
-        eval_along<PREC_GUARDED, 1, false, true>(p, ro, rd, sq, 1u, f32, unused, unused, cl,
-                                                 amb);
+        if (!p.gyro)
+          eval_along<PREC_GUARDED, 1, false, true>(p, ro, rd, sq, 1u, f32, unused, unused, cl,
+                                                   amb);
         const double ev = density64(p, ro[0] + rd[0] * sq[0], ro[1] + rd[1] * sq[0],
                                     ro[2] + rd[2] * sq[0], cl.idx, cl.n);
         wrong = ev != f32[0];
@@ -652,6 +578,14 @@ int launch_volume(const MarchParams& p, int res, double* dens, unsigned long lon
   return (int)hipGetLastError();
 }
 
+void launch_between(const MarchParams& p, int integrator, void* stream) {
+  const dim3 grid(std::min((p.defer_cap + 63u) / 64u, 8192u));
+  if (integrator == INT_HIERARCHICAL)
+    hipLaunchKernelGGL(march_hier_check_kernel, grid, dim3(64), 0, (hipStream_t)stream, p);
+  else
+    hipLaunchKernelGGL(march_resolve_kernel, grid, dim3(64), 0, (hipStream_t)stream, p);
+}
+
 int launch_march(const MarchParams& p, int precision, int integrator,
                  void* stream) {
   dim3 block(64);
@@ -669,7 +603,6 @@ int launch_march(const MarchParams& p, int precision, int integrator,
                          s, p);
   } else {
     if (integrator == INT_HIERARCHICAL && p.redo_list && !p.audit) {
-      const dim3 grid3(std::min((p.defer_cap + 63u) / 64u, 8192u));
       // 16384 one-wave groups for the redo pass's grid-stride: about one
       // batch of 64 rays each on C5 (891 k rays; 15.7 ms, 16.6 ms at 3072,
       // 24.5 ms at 1536), since a batch of such rays can take milliseconds
@@ -680,7 +613,7 @@ int launch_march(const MarchParams& p, int precision, int integrator,
         hipLaunchKernelGGL((march_hier_try_kernel<1, 2>), grid, block, 0, s, p);
       else
         hipLaunchKernelGGL((march_hier_try_kernel<2, 2>), grid, block, 0, s, p);
-      hipLaunchKernelGGL(march_hier_check_kernel, grid3, block, 0, s, p);
+      launch_between(p, integrator, stream);
       hipLaunchKernelGGL(march_hier_redo_kernel, grid2, block, 0, s, p);
     } else if (integrator == INT_HIERARCHICAL)
       hipLaunchKernelGGL((march_kernel<PREC_GUARDED, INT_HIERARCHICAL, kBlock>), grid,
@@ -688,15 +621,14 @@ int launch_march(const MarchParams& p, int precision, int integrator,
     else if (p.redo_list && !p.audit && !p.queue && (p.block == 1 || p.block == 2)) {
       // two passes and the resolve pass between them; the grids of the last
       // two stride over however many entries the first appended
-      const dim3 grid3(std::min((p.defer_cap + 63u) / 64u, 8192u));
       const dim3 grid2(std::min((p.redo_cap + 63u) / 64u, 1024u));
       if (p.block == 1) {
         hipLaunchKernelGGL(march_try_kernel<1>, grid, block, 0, s, p);
-        hipLaunchKernelGGL(march_resolve_kernel, grid3, block, 0, s, p);
+        launch_between(p, integrator, stream);
         hipLaunchKernelGGL(march_redo_kernel<1>, grid2, block, 0, s, p);
       } else {
         hipLaunchKernelGGL(march_try_kernel<2>, grid, block, 0, s, p);
-        hipLaunchKernelGGL(march_resolve_kernel, grid3, block, 0, s, p);
+        launch_between(p, integrator, stream);
         hipLaunchKernelGGL(march_redo_kernel<2>, grid2, block, 0, s, p);
       }
     } else if (p.block == 2 && p.queue)

@@ -133,6 +133,14 @@ struct MarchParams {
   int32_t line_cap;
   float line_eps;
   double line_seam;
+  // Gyroid march (gyroid_march.hpp): the gyroid's node index, 0 for the other
+  // marches; its density in the cell's collection; and, for the hierarchical
+  // integrator, the fine samples of each coarse step (at most 14).
+  int32_t gyro;
+  int32_t gyro_tanh;  // the chain is one tanh displacement
+  float gyro_band;    // guard band of | |g| - thickness | (gyroid_plan)
+  double gyro_rho;
+  const uint8_t* fine_n;
 };
 
 enum LineKind : int32_t { LINE_NONE = 0, LINE_COLL = 1, LINE_TESS = 2 };
@@ -266,6 +274,12 @@ int launch_volume(const MarchParams& p, int res, double* dens,
 // (simple integrator) in two passes: rays with an index that needs the FP64
 // evaluator are appended to it, and marched again by the second.
 int launch_line(const MarchParams& p, int integrator, void* stream);
+
+// Gyroid march of every pixel (p.gyro != 0), in two passes with p.redo_list.
+int launch_gyroid(const MarchParams& p, int integrator, void* stream);
+// The pass between the two of a two-pass march (march.hip): the resolve pass
+// of the simple integrator, the check pass of the hierarchical one.
+void launch_between(const MarchParams& p, int integrator, void* stream);
 
 // Launch on the given stream; returns hipError_t as int.
 int launch_march(const MarchParams& p, int precision, int integrator,

@@ -793,6 +793,7 @@ void flatten(const HNode& n, int depth, std::vector<DevNode>& out, Scene& s) {
       dn.f[4] = (float)n.b;
       dn.f[5] = (float)n.rho;
       dn.f[6] = (float)(1.0 / (n.a * 6.283185307179586476925286766559));
+      dn.f[7] = (float)(1.0 / (n.a * 6.283185307179586476925286766559) - (double)dn.f[6]);
       break;
     case K_VOXEL:
       dn.nx = n.nx;
