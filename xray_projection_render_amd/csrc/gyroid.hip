@@ -52,12 +52,33 @@ gyro_hier_try_kernel(MarchParams p) {
   try_finish<true>(p, q.v, q.i, q.j, q.valid, T, ts, rc);
 }
 
-template <int DEF, int INTEG, bool AUDIT>
+// The passes between (two_pass.hpp).  The first pass lists the membership it
+// used in bit 31.
+template <int DEF>
+__global__ __launch_bounds__(64) __attribute__((amdgpu_waves_per_eu(4))) void
+gyro_check_kernel(MarchParams p) {
+  two_pass_check(
+      p, [](int, int, int, bool) {},
+      [&](unsigned item, const double (&o)[3], const double (&d)[3], const double (&s)[1]) {
+        return gyro_exact<DEF>(p, o, d, s[0]) != ((item >> 31) != 0u);
+      });
+}
+template <int DEF>
+__global__ __launch_bounds__(64) __attribute__((amdgpu_waves_per_eu(4))) void
+gyro_resolve_kernel(MarchParams p) {
+  two_pass_resolve(
+      p, [](int, int, int, bool) {},
+      [&](const double (&o)[3], const double (&d)[3], double s) {
+        return gyro_exact<DEF>(p, o, d, s) ? p.gyro_rho : 0.0;
+      });
+}
+
+template <int DEF, int INTEG, bool AUDIT, int H = 1>
 __device__ __forceinline__ double gyro_T(const MarchParams& p, int v, int i, int j, bool valid,
                                          RayCounts& rc) {
   if constexpr (INTEG == INT_HIERARCHICAL) {
     __shared__ GyroRuns runs;
-    return gyro_T_hier<DEF, false, AUDIT>(p, v, i, j, valid, rc, nullptr, runs);
+    return gyro_T_hier<DEF, false, AUDIT, H>(p, v, i, j, valid, rc, nullptr, runs);
   } else {
     return gyro_T_simple<DEF, false, AUDIT>(p, v, i, j, valid, rc, nullptr);
   }
@@ -74,20 +95,29 @@ gyro_kernel(MarchParams p) {
   flush_counts(p.stats, rc);
 }
 
-// Last of the two passes: the listed rays, 64 per wave in list order.
+// Last of the two passes: the listed rays, 64 per wave in list order (simple),
+// or 4 with 16 lanes each (hierarchical: few rays, but with long chains of
+// visits and guard-band samples, so the pass lasts as long as its slowest
+// wave: 8074 rays of 25 M 1.18 -> 0.45 ms).
+template <int INTEG>
+struct GyroAgain {
+  static constexpr int lanes = INTEG == INT_HIERARCHICAL ? 16 : 1;
+};
 template <int DEF, int INTEG>
 __global__ __launch_bounds__(64) __attribute__((amdgpu_waves_per_eu(3))) void
 gyro_redo_kernel(MarchParams p) {
+  constexpr int H = GyroAgain<INTEG>::lanes;
+  constexpr unsigned rays = 64 / H;
   const unsigned n = min(p.counts[0], p.redo_cap);
   const unsigned rr = (unsigned)p.res * (unsigned)p.res;
   RayCounts rc;
-  for (unsigned base = blockIdx.x * 64u; base < n; base += gridDim.x * 64u) {
-    const unsigned e = base + threadIdx.x;
-    const bool valid = e < n;
+  for (unsigned base = blockIdx.x * rays; base < n; base += gridDim.x * rays) {
+    const unsigned e = base + threadIdx.x / H;
+    const bool valid = e < n && threadIdx.x % H == 0;
     const unsigned id = valid ? p.redo_list[e] : 0u;
     const unsigned v = id / rr, pix = id - v * rr;
     const int i = (int)(pix / (unsigned)p.res), j = (int)(pix - (unsigned)i * p.res);
-    const double T = gyro_T<DEF, INTEG, false>(p, (int)v, i, j, valid, rc);
+    const double T = gyro_T<DEF, INTEG, false, H>(p, (int)v, i, j, valid, rc);
     if (valid) store_pixel(p, (int)v, i, j, T);
   }
   flush_counts(p.stats, rc);
@@ -104,14 +134,15 @@ static int launch_def(const MarchParams& p, int integrator, hipStream_t s) {
   } else if (p.audit) {
     hipLaunchKernelGGL((gyro_kernel<DEF, INT_SIMPLE, true>), grid, block, 0, s, p);
   } else if (p.redo_list) {
-    const dim3 again(std::min((p.redo_cap + 63u) / 64u, 4096u));
+    const dim3 lists(std::min((p.defer_cap + 63u) / 64u, 8192u));
+    const dim3 again(std::min((p.redo_cap + 63u) / 64u, 8192u));
     if (hier) {
       hipLaunchKernelGGL((gyro_hier_try_kernel<DEF>), grid, block, 0, s, p);
-      launch_between(p, integrator, s);
+      hipLaunchKernelGGL((gyro_check_kernel<DEF>), lists, block, 0, s, p);
       hipLaunchKernelGGL((gyro_redo_kernel<DEF, INT_HIERARCHICAL>), again, block, 0, s, p);
     } else {
       hipLaunchKernelGGL((gyro_try_kernel<DEF>), grid, block, 0, s, p);
-      launch_between(p, integrator, s);
+      hipLaunchKernelGGL((gyro_resolve_kernel<DEF>), lists, block, 0, s, p);
       hipLaunchKernelGGL((gyro_redo_kernel<DEF, INT_SIMPLE>), again, block, 0, s, p);
     }
   } else if (hier) {

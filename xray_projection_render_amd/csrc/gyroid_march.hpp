@@ -30,6 +30,7 @@
 // of equal additions in a fixed order; the marches count and add at the end
 // (the same additions, hence the same bits, as march_ray.hpp).
 #pragma once
+#include "line_march.hpp"
 #include "march_ray.hpp"
 
 namespace xrp {
@@ -153,9 +154,30 @@ __device__ __forceinline__ GyroEval gyro_eval(const MarchParams& p, const GyroSc
   return o;
 }
 
-// FP64 membership at distance s along the ray.
-__device__ __forceinline__ bool gyro_exact(const MarchParams& p, const Ray& r, double s) {
-  return density64(p, r.o[0] + r.d[0] * s, r.o[1] + r.d[1] * s, r.o[2] + r.d[2] * s) != 0.0;
+// FP64 membership at distance s along the ray (density64's operations; the
+// constants through scalar loads).
+template <int DEF>
+__device__ __forceinline__ bool gyro_exact(const MarchParams& p, const double (&o)[3],
+                                           const double (&d)[3], double s) {
+  double x = o[0] + d[0] * s, y = o[1] + d[1] * s, z = o[2] + d[2] * s;
+  const LineNodes N = (LineNodes)line_uniform(p.nodes);
+  const LineDefs D = (LineDefs)line_uniform(p.defs);
+  if constexpr (DEF == GYRO_TANH) {
+    DevDeform f;
+    f.kind = D_TANH;
+    f.axis = D[0].axis;
+    f.src = D[0].src;
+    f.d[0] = D[0].d[0];
+    f.d[1] = D[0].d[1];
+    deform64(&f, 1, x, y, z);
+  } else if constexpr (DEF == GYRO_CHAIN) {
+    line_deform64(D, p.n_defs, x, y, z);
+  }
+  if (!line_wrap64(N, x, y, z)) return false;
+  double c[14];
+#pragma unroll
+  for (int q = 0; q < 5; ++q) c[q] = N[p.gyro].d[q];
+  return line_gyroid64(c, x, y, z);
 }
 
 // T + c added n times, in order.
@@ -210,7 +232,7 @@ __device__ __forceinline__ double gyro_T_simple(const MarchParams& p, int v, int
       if (!__ballot(go)) {
         if (!__ballot(wait)) break;
         if (wait) {
-          if (gyro_exact(p, r, p.s_table[k])) Ta += c;
+          if (gyro_exact<DEF>(p, r.o, r.d, p.s_table[k])) Ta += c;
           ++n_reeval;
           ++k;
           wait = false;
@@ -240,7 +262,7 @@ __device__ __forceinline__ double gyro_T_simple(const MarchParams& p, int v, int
         if (o.ahead >= 1.0f) m = min(o.ahead < 65536.0f ? (int)o.ahead : 65536, k_hi - k);
         if constexpr (AUDIT) {
           for (int q = 0; q <= m; ++q)
-            if (gyro_exact(p, r, p.s_table[k + q]) != o.in) ++n_miss;
+            if (gyro_exact<DEF>(p, r.o, r.d, p.s_table[k + q]) != o.in) ++n_miss;
         }
         if (o.in) hits += (unsigned)(m + 1);
         n_skip += (unsigned)m;
@@ -274,8 +296,10 @@ struct GyroRuns {
 // p.fine_n[n] of them) is 10 n + m + 1.  TRY: guard-band samples keep their FP32 densities
 // and are listed as march_T_hier<TRY> does, with the FP32 membership in bit
 // 31; otherwise the lanes wait for each other, and AUDIT compares, as in the
-// simple march.
-template <int DEF, bool TRY, bool AUDIT>
+// simple march.  H > 1: only every H-th lane has a ray, and the H lanes from
+// it on evaluate its next H coarse (or the step's next H fine) samples at
+// once: such rays run along the level, with many guard-band samples in a row.
+template <int DEF, bool TRY, bool AUDIT, int H = 1>
 __device__ __forceinline__ double gyro_T_hier(const MarchParams& p, int v, int i, int j,
                                               bool valid, RayCounts& rc, TryState* ts,
                                               GyroRuns& R) {
@@ -321,6 +345,11 @@ __device__ __forceinline__ double gyro_T_hier(const MarchParams& p, int v, int i
   int m = 0, m_hi = 0, nf = 0, inside = 0;
   float reach = 0.0f;
   bool wait = false;
+  // H > 1: bit q says whether sample known_at + q, fine ones of step n or
+  // (not known_fine) coarse ones, is inside
+  unsigned known = 0;
+  int known_at = -H;
+  bool known_fine = false;
   // adds the kept runs to T
   auto drain = [&]() {
     for (unsigned q = 0; q < runs; ++q) {
@@ -344,16 +373,16 @@ __device__ __forceinline__ double gyro_T_hier(const MarchParams& p, int v, int i
     }
     run += l;
   };
-  // fine sample q of step n, or its right end (q < 0)
-  auto at = [&](int q) {
-    if (q < 0) return p.s_table[n];
-    double s = (n == 0 ? p.smin : p.s_table[n - 1]) + dsf;
+  // fine sample q of step nn, or its right end (q < 0)
+  auto at = [&](int nn, int q) {
+    if (q < 0) return p.s_table[nn];
+    double s = (nn == 0 ? p.smin : p.s_table[nn - 1]) + dsf;
     for (int t = 0; t < q; ++t) s += dsf;
     return s;
   };
   auto audit = [&](int q, int end, bool in) {
     for (; q < end; ++q)
-      if (gyro_exact(p, r, at(q)) != in) ++n_miss;
+      if (gyro_exact<DEF>(p, r.o, r.d, at(n, q)) != in) ++n_miss;
   };
   for (;;) {
     bool go = n <= n_hi;
@@ -361,8 +390,30 @@ __device__ __forceinline__ double gyro_T_hier(const MarchParams& p, int v, int i
     if constexpr (!TRY) {
       if (!__ballot(go && !wait)) {
         if (!__ballot(wait)) break;
-        if (wait) {
-          ein = gyro_exact(p, r, at(fine ? m : -1));
+        if constexpr (H > 1) {
+          const int own = lane & ~(H - 1), h = lane & (H - 1);
+          double o[3], d[3];
+#pragma unroll
+          for (int c = 0; c < 3; ++c) {
+            o[c] = __shfl(r.o[c], own, 64);
+            d[c] = __shfl(r.d[c], own, 64);
+          }
+          const int f = __shfl(fine ? 1 : 0, own, 64), nn = __shfl(n, own, 64);
+          const int q = __shfl(fine ? m : n, own, 64) + h;
+          const int end = __shfl(fine ? nf : n_hi + 1, own, 64);
+          bool bit = false;
+          if (__shfl(wait ? 1 : 0, own, 64) && q < end)
+            bit = gyro_exact<DEF>(p, o, d, at(f ? nn : q, f ? q : -1));
+          const unsigned long long mask = __ballot(bit);
+          if (wait) {
+            known = (unsigned)(mask >> own) & ((1u << H) - 1u);
+            known_at = q;
+            known_fine = fine;
+            ein = known & 1u;
+            ++n_reeval;
+          }
+        } else if (wait) {
+          ein = gyro_exact<DEF>(p, r.o, r.d, at(n, fine ? m : -1));
           ++n_reeval;
         }
         exact = wait;
@@ -393,8 +444,14 @@ __device__ __forceinline__ double gyro_T_hier(const MarchParams& p, int v, int i
             continue;
           }
         } else {
-          wait = true;
-          continue;
+          const int q = (fine ? m : n) - known_at;
+          if (H > 1 && fine == known_fine && q >= 0 && q < H) {
+            o.in = (known >> q) & 1u;
+            ++n_reeval;
+          } else {
+            wait = true;
+            continue;
+          }
         }
       }
     }
@@ -437,6 +494,7 @@ __device__ __forceinline__ double gyro_T_hier(const MarchParams& p, int v, int i
         if (prev) close(run);
         run = 0;
         fine = false;
+        if (H > 1 && known_fine) known_at = -H;
       } else if (cur) {
         extend(1u);
       }
@@ -445,7 +503,7 @@ __device__ __forceinline__ double gyro_T_hier(const MarchParams& p, int v, int i
       if (f >= 1.0f) t = min(f < 65536.0f ? (int)f : 65536, n_hi - n);
       if constexpr (AUDIT) {
         for (int q = 1; q <= t; ++q)
-          if (gyro_exact(p, r, p.s_table[n + q]) != cur) ++n_miss;
+          if (gyro_exact<DEF>(p, r.o, r.d, p.s_table[n + q]) != cur) ++n_miss;
       }
       if (cur && t > 0) extend((unsigned)t);
       n_skip += (unsigned)t;

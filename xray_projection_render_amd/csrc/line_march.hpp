@@ -337,6 +337,24 @@ __device__ __forceinline__ unsigned long long line_uniform(const void* p) {
   return ((unsigned long long)hi << 32) | lo;
 }
 // One primitive's FP64 density at an object-space (cell-local) point.
+// gyroid64's operations (objects.go:1014-1032): inside the sheet.  The three
+// sines and cosines take turns in one copy of their code: it runs cold, and
+// fetching it costs more than running it.
+__device__ __forceinline__ bool line_gyroid64(const double (&k)[14], double X, double Y,
+                                              double Z) {
+  double q[3] = {(X - k[0]) / k[3], (Y - k[1]) / k[3], (Z - k[2]) / k[3]};
+  double s[3] = {0.0, 0.0, 0.0}, c[3] = {0.0, 0.0, 0.0};
+#pragma unroll 1
+  for (int a = 0; a < 3; ++a) {
+    double sa, ca;
+    sincos(q[0], &sa, &ca);
+    q[0] = q[1], q[1] = q[2];
+    s[0] = s[1], s[1] = s[2], s[2] = sa;
+    c[0] = c[1], c[1] = c[2], c[2] = ca;
+  }
+  const double g = s[0] * c[1] + s[1] * c[2] + s[2] * c[0];
+  return fabs(g) < k[4];
+}
 __device__ __forceinline__ double line_leaf64(LineNodes N, int c, double X, double Y, double Z) {
   DevNode k;
   k.kind = N[c].kind;
@@ -348,19 +366,16 @@ __device__ __forceinline__ double line_leaf64(LineNodes N, int c, double X, doub
     case K_PPED: return pped64(k, X, Y, Z);
     case K_CYL: return cyl64(k, X, Y, Z);
   }
-  // gyroid64's operations (objects.go:1014-1032)
-  X = (X - k.d[0]) / k.d[3];
-  Y = (Y - k.d[1]) / k.d[3];
-  Z = (Z - k.d[2]) / k.d[3];
-  const double g = sin(X) * cos(Y) + sin(Y) * cos(Z) + sin(Z) * cos(X);
-  return fabs(g) < k.d[4] ? k.d[5] : 0.0;
+  return line_gyroid64(k.d, X, Y, Z) ? k.d[5] : 0.0;
 }
-// The deformations line_plan admits (deform64's operations).
+// deform64's operations.
 __device__ __forceinline__ void line_deform64(LineDefs D, int nd, double& x, double& y,
                                               double& z) {
   for (int k = 0; k < nd; ++k) {
     DevDeform f;
     f.kind = D[k].kind;
+    f.axis = D[k].axis;
+    f.src = D[k].src;
 #pragma unroll
     for (int q = 0; q < 9; ++q) f.d[q] = D[k].d[q];
     deform64(&f, 1, x, y, z);

@@ -132,127 +132,26 @@ march_hier_try_kernel(MarchParams p) {
   try_finish<true>(p, v, i, j, valid, T, ts, rc);
 }
 
-// Check pass of the two-pass hierarchical march: 64 entries per wave
-// (grid-stride), their listed samples spread one per lane.  Each listed
-// sample, (nn << 4) | m, is at R[nn] for m = 15 and otherwise at
-// R[nn-1] + DS/10 plus m more additions of DS/10 (the
-// m-th sample of step nn's fine walk, main.go:180-186).  Its FP32 value,
-// which the first pass used, is computed again (it depends on the position
-// alone) and compared with its FP64 density; a ray with any that differs
-// goes to the redo list, whose pass overwrites its pixel, and its first
-// pass counts (after its items) are taken back from the stats.  Each wave
-// culls the root collection's children to its own 64 rays first.
-// One listed sample per lane rather than one ray per lane: on C5 18.6 ->
-// 11.3 ms (a wave ran as many rounds as its longest list, 1-14 samples).
+// Check pass (two_pass.hpp).  Each wave culls the root collection's children
+// to its own 64 rays first (a child culled is clear of every one of them in
+// FP32 and 0 in FP64, as in the first pass).  The FP32 value depends on the
+// position alone and is computed again.
 // 4 waves per SIMD (128 VGPRs, the FP64 evaluator's spilled): 11.2 ms, 11.4
 // at 3, 13.9 at 5 (one ray per lane: 24.5 ms at 2 waves, 18.5 at 4, 22.2
 // at 5).
 __global__ __launch_bounds__(64) __attribute__((amdgpu_waves_per_eu(4))) void
 march_hier_check_kernel(MarchParams p) {
-  const unsigned n = min(p.counts[1], p.defer_cap), nk = min(p.counts[2], p.k_cap);
-  const unsigned rr = (unsigned)p.res * (unsigned)p.res;
-  const double dsf = p.ds_fine;
-  unsigned long long reeval = 0, rays = 0, back_s = 0, back_f = 0, back_k = 0;
-  for (unsigned base = blockIdx.x * 64u; base < n; base += gridDim.x * 64u) {
-    const unsigned e = base + threadIdx.x;
-    unsigned cnt = 0u, k0 = 0u, id = 0u;
-    if (e < n) {
-      cnt = p.defer_cnt[e];
-      k0 = p.defer_kfirst[e];
-      if (k0 + cnt + 3u > nk) cnt = 0u;
-      // an entry marked empty (cnt 0, lists full) has no ray or k0 written
-      if (cnt != 0u)
-        id = p.defer_ray[e];
-      else
-        k0 = 0u;
-    }
-    const unsigned v = id / rr, pix = id - v * rr;
-    const int i = (int)(pix / (unsigned)p.res), j = (int)(pix - (unsigned)i * p.res);
-    // this wave's own cull list over its rays (a child culled here is clear
-    // of every one of them in FP32 and 0 in FP64, as in the first pass)
-    const Cull cl = wave_cull<1>(p, (int)v, i, j, cnt != 0u);
-    const Ray r = make_ray(p, p.views[p.view_offset + (int)v], i, j);
-    // The wave's listed samples, one per lane: lane l of round fb takes
-    // sample t = fb + l of the concatenated lists, owned by the ray (lane o)
-    // whose inclusive prefix sum of counts is the first above t.
-    unsigned incl = cnt;
-#pragma unroll
-    for (int off = 1; off < 64; off <<= 1) {
-      const unsigned u = __shfl_up(incl, off, 64);
-      if ((int)threadIdx.x >= off) incl += u;
-    }
-    const unsigned total = __builtin_amdgcn_readfirstlane(__shfl(incl, 63, 64));
-    unsigned long long bad = 0ull;  // lanes whose ray holds a wrong guess
-    for (unsigned fb = 0; fb < total; fb += 64u) {
-      const unsigned t = fb + threadIdx.x;
-      int o = 0;
-#pragma unroll
-      for (int step = 32; step >= 1; step >>= 1)
-        if (__shfl(incl, o + step - 1, 64) <= t) o += step;
-      const bool has = t < total;
-      const unsigned c = t - (__shfl(incl, o, 64) - __shfl(cnt, o, 64));
-      const unsigned ko = __shfl(k0, o, 64);
-      double ro[3], rd[3];
-#pragma unroll
-      for (int q = 0; q < 3; ++q) {
-        ro[q] = __shfl(r.o[q], o, 64);
-        rd[q] = __shfl(r.d[q], o, 64);
-      }
-      bool wrong = false;
-      if (has) {
-        const unsigned item = p.defer_k[ko + c], nn = (item & 0x7fffffffu) >> 4,
-                       m = item & 15u;
-        double sq[1];
-        if (m == 15u) {
-          sq[0] = p.s_table[nn];
-        } else {
-          sq[0] = (nn == 0 ? p.smin : p.s_table[nn - 1]) + dsf;
-          for (unsigned q = 0; q < m; ++q) sq[0] += dsf;
-        }
-        // the gyroid march lists the membership it used in bit 31
-        double f32[1] = {(item >> 31) ? p.gyro_rho : 0.0};
+  Cull cl;
+  two_pass_check(
+      p, [&](int v, int i, int j, bool valid) { cl = wave_cull<1>(p, v, i, j, valid); },
+      [&](unsigned, const double (&o)[3], const double (&d)[3], const double (&s)[1]) {
+        double f32[1];
         unsigned amb;
         unsigned long long unused = 0;
-        if (!p.gyro)
-          eval_along<PREC_GUARDED, 1, false, true>(p, ro, rd, sq, 1u, f32, unused, unused, cl,
-                                                   amb);
-        const double ev = density64(p, ro[0] + rd[0] * sq[0], ro[1] + rd[1] * sq[0],
-                                    ro[2] + rd[2] * sq[0], cl.idx, cl.n);
-        wrong = ev != f32[0];
-      }
-      for (unsigned long long w = __ballot(wrong); w; w &= w - 1ull) {
-        const int l = (int)__builtin_ctzll(w);
-        bad |= 1ull << __builtin_amdgcn_readlane(o, l);
-      }
-    }
-    if (cnt == 0u) continue;
-    const bool same = ((bad >> threadIdx.x) & 1ull) == 0ull;
-    if (same) {
-      reeval += cnt;
-      ++rays;
-    } else {
-      back_s += p.defer_k[k0 + cnt];
-      back_f += p.defer_k[k0 + cnt + 1];
-      back_k += p.defer_k[k0 + cnt + 2];
-      const unsigned at = atomicAdd(p.counts, 1u);
-      if (at < p.redo_cap)
-        p.redo_list[at] = id;
-      else
-        p.counts[3] = 1u;  // no room: the caller renders again in one pass
-    }
-  }
-  if (p.stats) {
-    const unsigned long long a = wave_sum(reeval), b = wave_sum(rays), c = wave_sum(back_s),
-                             d = wave_sum(back_f), f = wave_sum(back_k);
-    if (threadIdx.x == 0) {
-      if (a) atomicAdd(p.stats + ST_REEVAL, a);
-      if (b) atomicAdd(p.stats + ST_DEFERRED, b);
-      // the counts of rays marched again, taken back (mod 2^64)
-      if (c) atomicAdd(p.stats + ST_SAMPLES, 0ull - c);
-      if (d) atomicAdd(p.stats + ST_FINE, 0ull - d);
-      if (f) atomicAdd(p.stats + ST_SKIPPED, 0ull - f);
-    }
-  }
+        eval_along<PREC_GUARDED, 1, false, true>(p, o, d, s, 1u, f32, unused, unused, cl, amb);
+        return density64(p, o[0] + d[0] * s[0], o[1] + d[1] * s[0], o[2] + d[2] * s[0], cl.idx,
+                         cl.n) != f32[0];
+      });
 }
 
 // Second pass of the two-pass hierarchical march: the listed rays (stopped
@@ -275,92 +174,18 @@ march_hier_redo_kernel(MarchParams p) {
   flush_counts(p.stats, rc);
 }
 
-// Resolve pass: 64 entries of the first pass's lists per wave (grid-stride
-// over min(counts[1], defer_cap) entries), their deferred samples spread
-// one per lane.  Each is evaluated in FP64, its term (rho * dm) * ds staged
-// in LDS, and each entry's lane adds its own terms in sample order into Ta,
-// as the one-pass march sums its re-evaluated terms; the pixel is T + Ta.
-// The FP64 walks of a root collection visit the wave's own cull list.
-// A wave whose entries did not all fit wrote none of them but their count
-// 0 (its rays are in the redo list), and entries past the cap are not read.
+// Resolve pass (two_pass.hpp); the FP64 walks of a root collection visit the
+// wave's own cull list (a culled child is 0 along its rays).
 // 3 waves per SIMD: on C5 1.57 ms, 1.65 ms at 4, 2.80 ms at 6 (one entry
 // per lane, lists of 1-24 samples: 2.37 ms at 3 waves, 2.21 ms at 4).
 __global__ __launch_bounds__(64) __attribute__((amdgpu_waves_per_eu(3))) void
 march_resolve_kernel(MarchParams p) {
-  __shared__ double terms[64];
-  const unsigned n = min(p.counts[1], p.defer_cap), nk = min(p.counts[2], p.k_cap);
-  const unsigned rr = (unsigned)p.res * (unsigned)p.res;
-  const double ds = p.ds, dm = p.dm;
-  unsigned long long reeval = 0, rays = 0;
-  for (unsigned base = blockIdx.x * 64u; base < n; base += gridDim.x * 64u) {
-    const unsigned e = base + threadIdx.x;
-    unsigned cnt = 0u, k0 = 0u, id = 0u;
-    if (e < n) {
-      cnt = p.defer_cnt[e];
-      k0 = p.defer_kfirst[e];
-      if (k0 + cnt > nk) cnt = 0u;
-      // an entry marked empty (cnt 0, lists full) has no ray or k0 written
-      if (cnt != 0u)
-        id = p.defer_ray[e];
-      else
-        k0 = 0u;
-    }
-    const unsigned v = id / rr, pix = id - v * rr;
-    const int i = (int)(pix / (unsigned)p.res), j = (int)(pix - (unsigned)i * p.res);
-    // this wave's own cull list over its rays (a culled child is 0 along them)
-    const Cull cl = wave_cull<1>(p, (int)v, i, j, cnt != 0u);
-    const Ray r = make_ray(p, p.views[p.view_offset + (int)v], i, j);
-    // sample t of the concatenated lists belongs to the lane o whose
-    // inclusive prefix sum of counts is the first above t
-    unsigned incl = cnt;
-#pragma unroll
-    for (int off = 1; off < 64; off <<= 1) {
-      const unsigned u = __shfl_up(incl, off, 64);
-      if ((int)threadIdx.x >= off) incl += u;
-    }
-    const unsigned excl = incl - cnt;
-    const unsigned total = __builtin_amdgcn_readfirstlane(__shfl(incl, 63, 64));
-    double Ta = 0.0;
-    for (unsigned fb = 0; fb < total; fb += 64u) {
-      const unsigned t = fb + threadIdx.x;
-      int o = 0;
-#pragma unroll
-      for (int step = 32; step >= 1; step >>= 1)
-        if (__shfl(incl, o + step - 1, 64) <= t) o += step;
-      const unsigned c = t - __shfl(excl, o, 64);
-      const unsigned ko = __shfl(k0, o, 64);
-      double ro[3], rd[3];
-#pragma unroll
-      for (int q = 0; q < 3; ++q) {
-        ro[q] = __shfl(r.o[q], o, 64);
-        rd[q] = __shfl(r.d[q], o, 64);
-      }
-      double term = 0.0;
-      if (t < total) {
-        const double sk = p.s_table[p.defer_k[ko + c]];
-        const double ev = density64(p, ro[0] + rd[0] * sk, ro[1] + rd[1] * sk,
-                                    ro[2] + rd[2] * sk, cl.idx, cl.n);
-        term = (ev * dm) * ds;
-      }
-      terms[threadIdx.x] = term;
-      __syncthreads();
-      const unsigned lo = excl > fb ? excl : fb, hi = incl < fb + 64u ? incl : fb + 64u;
-      for (unsigned x = lo; x < hi; ++x) Ta += terms[x - fb];
-      __syncthreads();
-    }
-    if (cnt != 0u) {
-      store_pixel(p, (int)v, i, j, p.defer_T[e] + Ta);
-      reeval += cnt;
-      ++rays;
-    }
-  }
-  if (p.stats) {
-    const unsigned long long a = wave_sum(reeval), b = wave_sum(rays);
-    if (threadIdx.x == 0) {
-      if (a) atomicAdd(p.stats + ST_REEVAL, a);
-      if (b) atomicAdd(p.stats + ST_DEFERRED, b);
-    }
-  }
+  Cull cl;
+  two_pass_resolve(
+      p, [&](int v, int i, int j, bool valid) { cl = wave_cull<1>(p, v, i, j, valid); },
+      [&](const double (&o)[3], const double (&d)[3], double s) {
+        return density64(p, o[0] + d[0] * s, o[1] + d[1] * s, o[2] + d[2] * s, cl.idx, cl.n);
+      });
 }
 
 // Second pass: the rays the first pass listed, 64 per wave in list order
@@ -578,14 +403,6 @@ int launch_volume(const MarchParams& p, int res, double* dens, unsigned long lon
   return (int)hipGetLastError();
 }
 
-void launch_between(const MarchParams& p, int integrator, void* stream) {
-  const dim3 grid(std::min((p.defer_cap + 63u) / 64u, 8192u));
-  if (integrator == INT_HIERARCHICAL)
-    hipLaunchKernelGGL(march_hier_check_kernel, grid, dim3(64), 0, (hipStream_t)stream, p);
-  else
-    hipLaunchKernelGGL(march_resolve_kernel, grid, dim3(64), 0, (hipStream_t)stream, p);
-}
-
 int launch_march(const MarchParams& p, int precision, int integrator,
                  void* stream) {
   dim3 block(64);
@@ -603,6 +420,7 @@ int launch_march(const MarchParams& p, int precision, int integrator,
                          s, p);
   } else {
     if (integrator == INT_HIERARCHICAL && p.redo_list && !p.audit) {
+      const dim3 grid3(std::min((p.defer_cap + 63u) / 64u, 8192u));
       // 16384 one-wave groups for the redo pass's grid-stride: about one
       // batch of 64 rays each on C5 (891 k rays; 15.7 ms, 16.6 ms at 3072,
       // 24.5 ms at 1536), since a batch of such rays can take milliseconds
@@ -613,7 +431,7 @@ int launch_march(const MarchParams& p, int precision, int integrator,
         hipLaunchKernelGGL((march_hier_try_kernel<1, 2>), grid, block, 0, s, p);
       else
         hipLaunchKernelGGL((march_hier_try_kernel<2, 2>), grid, block, 0, s, p);
-      launch_between(p, integrator, stream);
+      hipLaunchKernelGGL(march_hier_check_kernel, grid3, block, 0, s, p);
       hipLaunchKernelGGL(march_hier_redo_kernel, grid2, block, 0, s, p);
     } else if (integrator == INT_HIERARCHICAL)
       hipLaunchKernelGGL((march_kernel<PREC_GUARDED, INT_HIERARCHICAL, kBlock>), grid,
@@ -621,14 +439,15 @@ int launch_march(const MarchParams& p, int precision, int integrator,
     else if (p.redo_list && !p.audit && !p.queue && (p.block == 1 || p.block == 2)) {
       // two passes and the resolve pass between them; the grids of the last
       // two stride over however many entries the first appended
+      const dim3 grid3(std::min((p.defer_cap + 63u) / 64u, 8192u));
       const dim3 grid2(std::min((p.redo_cap + 63u) / 64u, 1024u));
       if (p.block == 1) {
         hipLaunchKernelGGL(march_try_kernel<1>, grid, block, 0, s, p);
-        launch_between(p, integrator, stream);
+        hipLaunchKernelGGL(march_resolve_kernel, grid3, block, 0, s, p);
         hipLaunchKernelGGL(march_redo_kernel<1>, grid2, block, 0, s, p);
       } else {
         hipLaunchKernelGGL(march_try_kernel<2>, grid, block, 0, s, p);
-        launch_between(p, integrator, stream);
+        hipLaunchKernelGGL(march_resolve_kernel, grid3, block, 0, s, p);
         hipLaunchKernelGGL(march_redo_kernel<2>, grid2, block, 0, s, p);
       }
     } else if (p.block == 2 && p.queue)

@@ -277,9 +277,6 @@ int launch_line(const MarchParams& p, int integrator, void* stream);
 
 // Gyroid march of every pixel (p.gyro != 0), in two passes with p.redo_list.
 int launch_gyroid(const MarchParams& p, int integrator, void* stream);
-// The pass between the two of a two-pass march (march.hip): the resolve pass
-// of the simple integrator, the check pass of the hierarchical one.
-void launch_between(const MarchParams& p, int integrator, void* stream);
 
 // Launch on the given stream; returns hipError_t as int.
 int launch_march(const MarchParams& p, int precision, int integrator,
