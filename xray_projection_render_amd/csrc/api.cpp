@@ -1106,7 +1106,9 @@ int render_core(xrp_context* ctx, xrp_scene* sc, const RenderJob& job,
   const size_t b_nodes = pl.nodes.size() * sizeof(DevNode);
   const size_t b_defs = s.ddefs.size() * sizeof(DevDeform);
   const size_t b_views = (size_t)nv * sizeof(DevView);
-  const size_t b_stats = ST_COUNT * sizeof(unsigned long long);
+  const uint32_t copies = fixed ? 1 : kStatCopies;
+  const size_t b_stats =
+      ((size_t)(copies - 1) * kStatStride + ST_COUNT) * sizeof(unsigned long long);
   const size_t o_defs = align(b_nodes), o_views = o_defs + align(std::max<size_t>(b_defs, 1));
   const size_t o_stats = o_views + align(b_views);
   // zeroed list counters of the two-pass march, one per launch
@@ -1165,6 +1167,7 @@ int render_core(xrp_context* ctx, xrp_scene* sc, const RenderJob& job,
   mp.views = (const DevView*)(db + o_views);
   mp.s_table = fixed ? (const double*)(db + o_table) : (const double*)ctx->table.p;
   mp.stats = (unsigned long long*)(db + o_stats);
+  mp.stat_mask = copies - 1;
   if (fixed || (hier && ctx->table_fine_most > 14)) mp.gyro = 0;
   if (mp.gyro && hier) mp.fine_n = (const uint8_t*)(mp.s_table + pl.table.size());
   (void)res;
@@ -1218,8 +1221,9 @@ int render_core(xrp_context* ctx, xrp_scene* sc, const RenderJob& job,
   const size_t b_back = two_pass ? o_ctr + b_ctr - o_stats : b_stats;
   HIPCHK(hipMemcpyAsync(hstp, mp.stats, b_back, hipMemcpyDeviceToHost, ctx->stream));
   HIPCHK(hipStreamSynchronize(ctx->stream));
-  unsigned long long hst[ST_COUNT];
-  std::memcpy(hst, hstp, sizeof hst);
+  unsigned long long hst[ST_COUNT] = {};
+  for (uint32_t c = 0; c < copies; ++c)
+    for (int k = 0; k < ST_COUNT; ++k) hst[k] += hstp[c * kStatStride + k];
   uint64_t redo_rays = 0;
   bool overflow = false;
   for (int c = 0; two_pass && c < n_chunks; ++c) {

@@ -764,4 +764,23 @@ __device__ __forceinline__ unsigned long long wave_sum(unsigned long long v) {
   return v;
 }
 
+// This block's copy of the launch's counters, or null.
+__device__ __forceinline__ unsigned long long* stat_slot(const MarchParams& p) {
+  return p.stats ? p.stats + (size_t)(blockIdx.x & p.stat_mask) * kStatStride : nullptr;
+}
+
+// Sum over the wave (every lane active), 32-bit steps where they suffice.
+__device__ __forceinline__ unsigned long long wave_total(unsigned long long v) {
+  if (!__ballot(v != 0ull)) return 0ull;
+  if (__ballot((v >> 26) != 0ull)) return wave_sum(v);
+  int x = (int)(unsigned)v;
+  x += __builtin_amdgcn_update_dpp(0, x, 0x111, 0xf, 0xf, true);   // row_shr:1
+  x += __builtin_amdgcn_update_dpp(0, x, 0x112, 0xf, 0xf, true);   // row_shr:2
+  x += __builtin_amdgcn_update_dpp(0, x, 0x114, 0xf, 0xf, true);   // row_shr:4
+  x += __builtin_amdgcn_update_dpp(0, x, 0x118, 0xf, 0xf, true);   // row_shr:8
+  x += __builtin_amdgcn_update_dpp(0, x, 0x142, 0xa, 0xf, false);  // row_bcast:15
+  x += __builtin_amdgcn_update_dpp(0, x, 0x143, 0xc, 0xf, false);  // row_bcast:31
+  return (unsigned)__builtin_amdgcn_readlane(x, 63);
+}
+
 }  // namespace xrp

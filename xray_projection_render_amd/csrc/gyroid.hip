@@ -92,7 +92,7 @@ gyro_kernel(MarchParams p) {
   RayCounts rc;
   const double T = gyro_T<DEF, INTEG, AUDIT>(p, q.v, q.i, q.j, q.valid, rc);
   if (q.valid) store_pixel(p, q.v, q.i, q.j, T);
-  flush_counts(p.stats, rc);
+  flush_counts(p, rc);
 }
 
 // Last of the two passes: the listed rays, 64 per wave in list order (simple),
@@ -120,7 +120,7 @@ gyro_redo_kernel(MarchParams p) {
     const double T = gyro_T<DEF, INTEG, false, H>(p, (int)v, i, j, valid, rc);
     if (valid) store_pixel(p, (int)v, i, j, T);
   }
-  flush_counts(p.stats, rc);
+  flush_counts(p, rc);
 }
 
 template <int DEF>

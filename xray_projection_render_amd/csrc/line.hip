@@ -82,7 +82,7 @@ line_kernel(MarchParams p) {
   RayCounts rc;
   const double T = line_pixel_T<INTEG, AUDIT, KIND>(p, q.v, q.i, q.j, q.valid, S, p.line_cap, rc);
   if (q.valid) store_pixel(p, q.v, q.i, q.j, T);
-  flush_counts(p.stats, rc);
+  flush_counts(p, rc);
 }
 
 // First pass of the two-pass form: the stopped rays are appended to
@@ -111,7 +111,7 @@ line_try_kernel(MarchParams p) {
         p.counts[3] = 1u;  // no room: the caller renders again in one pass
     }
   }
-  flush_counts(p.stats, rc);
+  flush_counts(p, rc);
 }
 
 // Second pass: one listed ray per wave (grid-stride).
@@ -125,7 +125,7 @@ __global__ __launch_bounds__(64) void line_redo_kernel(MarchParams p) {
     const double T = line_T_exact<INT_SIMPLE>(p, (int)v, i, j, 0, rc);
     if (threadIdx.x == 0) store_pixel(p, (int)v, i, j, T);
   }
-  flush_counts(p.stats, rc);
+  flush_counts(p, rc);
 }
 
 // Batched form: the items of one group (batch.hip), every job of it with

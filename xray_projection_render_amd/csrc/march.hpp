@@ -31,6 +31,14 @@ enum StatSlot {
   ST_COUNT = 9
 };
 
+// The counters' copies of a per-scene render.  Every wave adds two to five
+// counters as it ends, and an add to a line that another wave is adding to
+// takes about 4 ns, so that one copy bounded launches of many short waves (60
+// primitives, 16 x 512^2, hierarchical: 0.50 ms against 0.33 ms without
+// counters).
+constexpr int kStatStride = 16;
+constexpr uint32_t kStatCopies = 64;
+
 struct MarchParams {
   const DevNode* nodes;
   const DevDeform* defs;
@@ -38,6 +46,9 @@ struct MarchParams {
   const double* s_table;   // simple: s_k; hierarchical: coarse right_n
   float* out;              // [view][i][j] f32 transmittance
   unsigned long long* stats;
+  // Copies of the counters less one (a power of two less one), each on a line
+  // of its own (kStatStride words): block b adds to copy b & stat_mask.
+  uint32_t stat_mask;
   int32_t n_defs;
   int32_t n_views;
   int32_t res;

@@ -900,12 +900,13 @@ __device__ __forceinline__ void march_ray(const MarchParams& p, int v, int i, in
   if (valid) store_pixel(p, v, i, j, T);
 }
 
-// Wave-reduced counters into a launch's stats slots (lane 0 writes).
-__device__ __forceinline__ void flush_counts(unsigned long long* stats, const RayCounts& rc) {
+// Wave-reduced counters into the launch's counters (lane 0 writes).
+__device__ __forceinline__ void flush_counts(const MarchParams& p, const RayCounts& rc) {
+  unsigned long long* stats = stat_slot(p);
   if (!stats) return;
-  unsigned long long a = wave_sum(rc.samples), b = wave_sum(rc.reeval),
-                     c = wave_sum(rc.miss), d = wave_sum(rc.fine),
-                     e = wave_sum(rc.skipped);
+  unsigned long long a = wave_total(rc.samples), b = wave_total(rc.reeval),
+                     c = wave_total(rc.miss), d = wave_total(rc.fine),
+                     e = wave_total(rc.skipped);
   if ((threadIdx.x & 63) == 0) {
     if (a) atomicAdd(stats + ST_SAMPLES, a);
     if (b) atomicAdd(stats + ST_REEVAL, b);

@@ -80,7 +80,7 @@ __device__ __forceinline__ void try_finish(const MarchParams& p, int v, int i, i
         p.counts[3] = 1u;  // no room: the caller renders again in one pass
     }
   }
-  flush_counts(p.stats, rc);
+  flush_counts(p, rc);
 }
 
 // Check pass of the two-pass hierarchical march: 64 entries per wave
@@ -178,16 +178,16 @@ __device__ __forceinline__ void two_pass_check(const MarchParams& p, Begin begin
         p.counts[3] = 1u;  // no room: the caller renders again in one pass
     }
   }
-  if (p.stats) {
-    const unsigned long long a = wave_sum(reeval), b = wave_sum(rays), c = wave_sum(back_s),
-                             d = wave_sum(back_f), f = wave_sum(back_k);
+  if (unsigned long long* stats = stat_slot(p)) {
+    const unsigned long long a = wave_total(reeval), b = wave_total(rays), c = wave_total(back_s),
+                             d = wave_total(back_f), f = wave_total(back_k);
     if (threadIdx.x == 0) {
-      if (a) atomicAdd(p.stats + ST_REEVAL, a);
-      if (b) atomicAdd(p.stats + ST_DEFERRED, b);
+      if (a) atomicAdd(stats + ST_REEVAL, a);
+      if (b) atomicAdd(stats + ST_DEFERRED, b);
       // the counts of rays marched again, taken back (mod 2^64)
-      if (c) atomicAdd(p.stats + ST_SAMPLES, 0ull - c);
-      if (d) atomicAdd(p.stats + ST_FINE, 0ull - d);
-      if (f) atomicAdd(p.stats + ST_SKIPPED, 0ull - f);
+      if (c) atomicAdd(stats + ST_SAMPLES, 0ull - c);
+      if (d) atomicAdd(stats + ST_FINE, 0ull - d);
+      if (f) atomicAdd(stats + ST_SKIPPED, 0ull - f);
     }
   }
 }
@@ -267,11 +267,11 @@ __device__ __forceinline__ void two_pass_resolve(const MarchParams& p, Begin beg
       ++rays;
     }
   }
-  if (p.stats) {
-    const unsigned long long a = wave_sum(reeval), b = wave_sum(rays);
+  if (unsigned long long* stats = stat_slot(p)) {
+    const unsigned long long a = wave_total(reeval), b = wave_total(rays);
     if (threadIdx.x == 0) {
-      if (a) atomicAdd(p.stats + ST_REEVAL, a);
-      if (b) atomicAdd(p.stats + ST_DEFERRED, b);
+      if (a) atomicAdd(stats + ST_REEVAL, a);
+      if (b) atomicAdd(stats + ST_DEFERRED, b);
     }
   }
 }

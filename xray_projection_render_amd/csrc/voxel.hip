@@ -479,9 +479,9 @@ __device__ __forceinline__ void voxel_body(const MarchParams& p) {
   }
   if (valid)
     store_pixel(p, blockIdx.y, i, j, T);
-  if (p.stats) {
-    unsigned long long a = wave_sum(kb >= ka ? (unsigned long long)(kb - ka + 1) : 0ull);
-    if (lane == 0 && a) atomicAdd(p.stats + ST_SAMPLES, a);
+  if (unsigned long long* stats = stat_slot(p)) {
+    unsigned long long a = wave_total(kb >= ka ? (unsigned long long)(kb - ka + 1) : 0ull);
+    if (lane == 0 && a) atomicAdd(stats + ST_SAMPLES, a);
   }
 }
 
@@ -699,14 +699,14 @@ __global__ __launch_bounds__(64) void voxel_lds_kernel(MarchParams p) {
   }
   if (valid)
     store_pixel(p, blockIdx.y, i, j, T);
-  if (p.stats) {
-    unsigned long long a = wave_sum(kb >= ka ? (unsigned long long)(kb - ka + 1) : 0ull);
+  if (unsigned long long* stats = stat_slot(p)) {
+    unsigned long long a = wave_total(kb >= ka ? (unsigned long long)(kb - ka + 1) : 0ull);
     if (lane == 0) {
-      if (a) atomicAdd(p.stats + ST_SAMPLES, a);
+      if (a) atomicAdd(stats + ST_SAMPLES, a);
       // wave-uniform staging counters
-      if (n_chunks) atomicAdd(p.stats + ST_STAGED_CHUNKS, n_chunks);
-      if (n_staged) atomicAdd(p.stats + ST_STAGED_VOXELS, n_staged);
-      if (n_fallback) atomicAdd(p.stats + ST_FALLBACK_CHUNKS, n_fallback);
+      if (n_chunks) atomicAdd(stats + ST_STAGED_CHUNKS, n_chunks);
+      if (n_staged) atomicAdd(stats + ST_STAGED_VOXELS, n_staged);
+      if (n_fallback) atomicAdd(stats + ST_FALLBACK_CHUNKS, n_fallback);
     }
   }
 }
