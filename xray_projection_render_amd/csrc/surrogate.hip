@@ -15,6 +15,7 @@
 // 8+2g and 9+2g: every lane encodes four levels of its sample.
 #include <hip/hip_runtime.h>
 
+#include <algorithm>
 #include <cmath>
 
 #include "eval_device.hpp"
@@ -30,6 +31,15 @@ __device__ __forceinline__ short f2bf(float f) {  // round to nearest even
   unsigned u = __float_as_uint(f);
   u += 0x7fffu + ((u >> 16) & 1u);
   return (short)(u >> 16);
+}
+// f2bf of four finite values (v_cvt_pk_bf16_f32, round to nearest even)
+__device__ __forceinline__ bf16x4 f2bf4(float a, float b, float c, float d) {
+  typedef float f2 __attribute__((ext_vector_type(2)));
+  typedef __bf16 h2 __attribute__((ext_vector_type(2)));
+  typedef short s2 __attribute__((ext_vector_type(2)));
+  const s2 p = __builtin_bit_cast(s2, __builtin_convertvector((f2{a, b}), h2));
+  const s2 q = __builtin_bit_cast(s2, __builtin_convertvector((f2{c, d}), h2));
+  return bf16x4{p[0], p[1], q[0], q[1]};
 }
 __device__ __forceinline__ float bf2f(unsigned h) { return __uint_as_float(h << 16); }
 
@@ -111,28 +121,6 @@ __device__ __forceinline__ void encode_f32(const SurNet& net, int g, float ux, f
       const float2 e = tab[(size_t)l * T + c.idx[k]];
       f0 = fmaf(c.w[k], e.x, f0);
       f1 = fmaf(c.w[k], e.y, f1);
-    }
-    feat[2 * q] = f0;
-    feat[2 * q + 1] = f1;
-  }
-}
-
-// The same from the packed BF16 inference tables (one dword per entry).
-__device__ __forceinline__ void encode_bf16(const SurNet& net, int g, float ux, float uy,
-                                            float uz, float (&feat)[8]) {
-  const uint32_t T = 1u << net.log2_table, tmask = T - 1u;
-#pragma unroll
-  for (int q = 0; q < 4; ++q) {
-    const int l = lane_level(g, q);
-    const int N = net.res[l];
-    const LevelCell c = level_cell(N, tmask, level_dense(N, net.log2_table), ux, uy, uz);
-    const uint32_t* tab = net.table_bf16 + (size_t)l * T;
-    float f0 = 0.0f, f1 = 0.0f;
-#pragma unroll
-    for (int k = 0; k < 8; ++k) {
-      const uint32_t e = tab[c.idx[k]];
-      f0 = fmaf(c.w[k], bf2f(e & 0xffffu), f0);
-      f1 = fmaf(c.w[k], bf2f(e >> 16), f1);
     }
     feat[2 * q] = f0;
     feat[2 * q + 1] = f1;
@@ -543,87 +531,257 @@ __device__ __forceinline__ bool sur_domain(const SurNet& net, float x, float y, 
   return ux >= 0.0f && ux <= 1.0f && uy >= 0.0f && uy <= 1.0f && uz >= 0.0f && uz <= 1.0f;
 }
 
-// One wave per workgroup (16 rays, a 4x4 pixel tile, each with its own LDS
-// copy of the weights): waves whose rays end early free their slot at once
-// (5 % faster than 8x8 tiles of four waves).
-__global__ __launch_bounds__(64) void sur_render_kernel(SurNet net, MarchParams p,
-                                                         double ds_sur, long K) {
-  __shared__ SurFwdLds F;
-  const SurOffsets off = sur_offsets(net.log2_table);
-  const float* P = net.params;
-  stage_fwd(F, P + off.W1, P + off.W2);
-  __syncthreads();
-  const float* b1 = P + off.b1;
-  const float* b2 = P + off.b2;
-  const float* w3 = P + off.w3;
-  const float b3 = P[off.b3];
+// The march's operands in LDS: the weights' and, per unit tile and lane group,
+// the four biases (of both layers) and output weights that group's lanes use.
+constexpr uint32_t kSurLdsEntries = 37600;  // 147 KiB
+struct SurMarchLds {
+  SurFwdLds F;
+  f32x4 b1[4][4], b2[4][4], w3[4][4];
+  uint32_t tab[kSurLdsEntries];  // tables of the first levels, as many as fit
+};
+static_assert(sizeof(SurMarchLds) <= 160 * 1024, "one workgroup a CU");
 
-  const int lane = threadIdx.x & 63;
-  const int s = lane & 15, g = lane >> 4;
-  const int tiles_j = (p.res + 3) >> 2;
-  const int ti = blockIdx.x / tiles_j, tj = blockIdx.x - ti * tiles_j;
-  const int i = ti * 4 + (s >> 2);
-  const int j = tj * 4 + (s & 3);
-  const int v = blockIdx.y;
-  const bool valid = i < p.res && j < p.res;
+// A lane's four hash levels: cells per axis, the strides of y and z (of a
+// dense level's grid, or the hash's factors) and the first table entry, in
+// LDS or in the level's global table.
+struct SurLevels {
+  float n[4];
+  uint32_t y[4], z[4], first[4];
+  bool dense[4], lds[4];
+};
 
-  long k_lo = 1, k_hi = 0;
-  Ray r;
-  r.o[0] = r.o[1] = r.o[2] = 0.0;
-  r.d[0] = r.d[1] = r.d[2] = 0.0;
-  if (valid) {
-    r = make_ray(p, p.views[p.view_offset + v], i, j);
-    double t_in, t_out;
-    if (clip_ray(p, r, t_in, t_out)) {
-      double a = floor((t_in - p.smin) / ds_sur - 0.5) - 1.0;
-      double b = ceil((t_out - p.smin) / ds_sur - 0.5) + 1.0;
-      k_lo = a > 0.0 ? (long)a : 0;
-      k_hi = b < (double)(K - 1) ? (long)b : K - 1;
+// Entries that level l's cells reach.
+__device__ __forceinline__ uint32_t sur_entries(const SurNet& net, int l) {
+  const uint32_t n1 = (uint32_t)net.res[l] + 1u;
+  return level_dense(net.res[l], net.log2_table) ? n1 * n1 * n1 : 1u << net.log2_table;
+}
+
+__device__ __forceinline__ SurLevels sur_levels(const SurNet& net, int g, int n_lds) {
+  SurLevels L;
+#pragma unroll
+  for (int q = 0; q < 4; ++q) {
+    const int l = lane_level(g, q), N = net.res[l];
+    L.dense[q] = level_dense(N, net.log2_table);
+    L.n[q] = (float)N;
+    L.y[q] = L.dense[q] ? (uint32_t)N + 1u : 2654435761u;
+    L.z[q] = L.dense[q] ? ((uint32_t)N + 1u) * ((uint32_t)N + 1u) : 805459861u;
+    L.lds[q] = l < n_lds;
+    L.first[q] = (uint32_t)l << net.log2_table;
+    if (L.lds[q]) {
+      L.first[q] = 0;
+      for (int k = 0; k < l; ++k) L.first[q] += sur_entries(net, k);
     }
   }
-  long wlo = k_lo, whi = k_hi;
-  // the union of the wave's sample ranges (empty ranges have lo > hi)
-  if (k_lo > k_hi) {
-    wlo = 0x7fffffffffffL;
-    whi = -1;
+  return L;
+}
+
+// The lane's features at u in [0, 1]^3 from the packed BF16 tables: all 32
+// gathers first, then the sums, whose terms and order are encode_f32's.
+__device__ __forceinline__ void encode_bf16(const uint32_t* __restrict__ tab,
+                                            const uint32_t* lds_tab, uint32_t tmask,
+                                            const SurLevels& L, float ux, float uy, float uz,
+                                            float (&feat)[8]) {
+  uint32_t e[4][8];
+  float w[4][3];
+#pragma unroll
+  for (int q = 0; q < 4; ++q) {
+    const float gx = ux * L.n[q], gy = uy * L.n[q], gz = uz * L.n[q];
+    const float top = L.n[q] - 1.0f;
+    const float fx = fminf(floorf(gx), top), fy = fminf(floorf(gy), top),
+                fz = fminf(floorf(gz), top);
+    w[q][0] = gx - fx, w[q][1] = gy - fy, w[q][2] = gz - fz;
+    const uint32_t x = (uint32_t)fx, y = (uint32_t)fy * L.y[q], z = (uint32_t)fz * L.z[q];
+    uint32_t at[8];
+#pragma unroll
+    for (int k = 0; k < 8; ++k) {
+      const uint32_t cx = x + ((k >> 2) & 1), cy = y + ((k >> 1) & 1) * L.y[q],
+                     cz = z + (k & 1) * L.z[q];
+      at[k] = L.first[q] + (L.dense[q] ? cx + cy + cz : (cx ^ cy ^ cz) & tmask);
+    }
+    if (L.lds[q]) {
+#pragma unroll
+      for (int k = 0; k < 8; ++k) e[q][k] = lds_tab[at[k]];
+    } else {
+      // 32-bit byte offsets (16 levels of at most 2^24 entries); the two
+      // corners along x, mostly of one line, one after the other
+#pragma unroll
+      for (int j = 0; j < 8; ++j) {
+        const int k = (j >> 1) | ((j & 1) << 2);
+        e[q][k] = *(const uint32_t*)((const char*)tab + (at[k] << 2));
+      }
+    }
   }
 #pragma unroll
-  for (int o = 1; o < 64; o <<= 1) {
-    wlo = min(wlo, (long)__shfl_xor(wlo, o, 64));
-    whi = max(whi, (long)__shfl_xor(whi, o, 64));
+  for (int q = 0; q < 4; ++q) {
+    float f0 = 0.0f, f1 = 0.0f;
+#pragma unroll
+    for (int k = 0; k < 8; ++k) {
+      const float c = ((k & 4) ? w[q][0] : 1.0f - w[q][0]) *
+                      ((k & 2) ? w[q][1] : 1.0f - w[q][1]) *
+                      ((k & 1) ? w[q][2] : 1.0f - w[q][2]);
+      f0 = fmaf(c, bf2f(e[q][k] & 0xffffu), f0);
+      f1 = fmaf(c, bf2f(e[q][k] >> 16), f1);
+    }
+    feat[2 * q] = f0;
+    feat[2 * q + 1] = f1;
   }
-  if (p.stats && lane == 0 && whi >= wlo)
-    atomicAdd(p.stats + ST_SAMPLES, (unsigned long long)(whi - wlo + 1) * 16ull);
-  float acc = 0.0f, comp = 0.0f;
-  const float d0 = (float)r.d[0], d1 = (float)r.d[1], d2 = (float)r.d[2];
+}
+
+// mlp_forward with its constants in LDS and no activations kept.
+__device__ __forceinline__ float mlp_density(const SurMarchLds& L, float b3, int lane,
+                                             const float (&feat)[8]) {
+  const int g = lane >> 4;
+  const bf16x4 x0 = f2bf4(feat[0], feat[1], feat[2], feat[3]);
+  const bf16x4 x1 = f2bf4(feat[4], feat[5], feat[6], feat[7]);
+  bf16x4 h[4];
+#pragma unroll
+  for (int mt = 0; mt < 4; ++mt) {
+    f32x4 acc = {0.0f, 0.0f, 0.0f, 0.0f};
+    acc = mfma16(L.F.a1[mt][0][lane], x0, acc);
+    acc = mfma16(L.F.a1[mt][1][lane], x1, acc);
+    const f32x4 b = L.b1[mt][g];
+    h[mt] = f2bf4(fmaxf(acc[0] + b[0], 0.0f), fmaxf(acc[1] + b[1], 0.0f),
+                  fmaxf(acc[2] + b[2], 0.0f), fmaxf(acc[3] + b[3], 0.0f));
+  }
+  float part = 0.0f;
+#pragma unroll
+  for (int mt = 0; mt < 4; ++mt) {
+    f32x4 acc = {0.0f, 0.0f, 0.0f, 0.0f};
+#pragma unroll
+    for (int kb = 0; kb < 4; ++kb) acc = mfma16(L.F.a2[mt][kb][lane], h[kb], acc);
+    const f32x4 b = L.b2[mt][g], w = L.w3[mt][g];
+#pragma unroll
+    for (int i = 0; i < 4; ++i) part = fmaf(w[i], fmaxf(acc[i] + b[i], 0.0f), part);
+  }
+  part += __shfl_xor(part, 16, 64);
+  part += __shfl_xor(part, 32, 64);
+  return 1.0f / (1.0f + expf(-(part + b3)));
+}
+
+// One workgroup a CU, which stays for the launch: it stages the weights and
+// tables once, and its waves take tiles (16 rays, 4x4 pixels) from the counter
+// p.counts until none is left.
+//
+// The gathers bound it: 64 lines of a step's 128 corners are distinct for each
+// sample (fine cells are smaller than the pixel spacing), and L1 and L2 are
+// smaller than what the waves have in flight and the tables.  Of 2^17-entry
+// tables (8 MiB), 4 x 256^2 rays at step 0.008: 3.18 ms with one wave per
+// workgroup and the corners in index order; 3.3 with this workgroup's operands
+// in LDS; 2.57 with the first levels' tables in LDS as well (three of 16 levels'
+// requests gone, 2 waves a SIMD); 2.1 with the corners along x, mostly of one
+// line, loaded one after the other (L2 requests 340 -> 212 M).  2 waves a SIMD:
+// 2.11 ms; 2.31 at 1, 2.48 at 3 and 2.57 at 4, which evict each other's lines.
+// One 8-byte load for an aligned pair of corners: 2.58 ms.
+constexpr int kSurMarchWaves = 8;
+constexpr int kSurGroups = 256;
+
+__global__ __launch_bounds__(64 * kSurMarchWaves)
+    __attribute__((amdgpu_waves_per_eu(2))) void sur_render_kernel(SurNet net, MarchParams p,
+                                                                   double ds_sur, long K,
+                                                                   unsigned n_tiles) {
+  __shared__ SurMarchLds L;
+  const SurOffsets off = sur_offsets(net.log2_table);
+  const float* P = net.params;
+  stage_fwd(L.F, P + off.W1, P + off.W2);
+  if (threadIdx.x < 64) {
+    ((float*)L.b1)[threadIdx.x] = P[off.b1 + threadIdx.x];
+    ((float*)L.b2)[threadIdx.x] = P[off.b2 + threadIdx.x];
+    ((float*)L.w3)[threadIdx.x] = P[off.w3 + threadIdx.x];
+  }
+  int n_lds = 0;
+  for (uint32_t at = 0; n_lds < kSurLevels; ++n_lds) {
+    const uint32_t n = sur_entries(net, n_lds);
+    if (n > kSurLdsEntries - at) break;
+    const uint32_t* t = net.table_bf16 + ((size_t)n_lds << net.log2_table);
+    for (uint32_t e = threadIdx.x; e < n; e += blockDim.x) L.tab[at + e] = t[e];
+    at += n;
+  }
+  __syncthreads();
+  const float b3 = P[off.b3];
+  const int lane = threadIdx.x & 63;
+  const int s = lane & 15, g = lane >> 4;
+  const SurLevels levels = sur_levels(net, g, n_lds);
+  const uint32_t tmask = (1u << net.log2_table) - 1u;
+  const int tiles_j = (p.res + 3) >> 2;
+  const unsigned per_view = (unsigned)tiles_j * (unsigned)tiles_j;
   const float dsf = (float)ds_sur;
-  for (long k0 = wlo; k0 <= whi; k0 += kChunk) {
-    const double sa = p.smin + ((double)k0 + 0.5) * ds_sur;
-    const float a0 = (float)(r.o[0] + r.d[0] * sa), a1 = (float)(r.o[1] + r.d[1] * sa),
-                a2 = (float)(r.o[2] + r.d[2] * sa);
-    const int n = (int)min((long)kChunk, whi - k0 + 1);
-    for (int jj = 0; jj < n; ++jj) {
-      const float sj = (float)jj * dsf;
-      float x = fmaf(d0, sj, a0), y = fmaf(d1, sj, a1), z = fmaf(d2, sj, a2);
-      deform32(p.defs, p.n_defs, x, y, z);
-      float ux = 0.5f, uy = 0.5f, uz = 0.5f;
-      const long k = k0 + jj;
-      const bool in = sur_domain(net, x, y, z, ux, uy, uz) && k >= k_lo && k <= k_hi;
-      float feat[8];
-      encode_bf16(net, g, in ? ux : 0.5f, in ? uy : 0.5f, in ? uz : 0.5f, feat);
-      SurAct act;
-      const float dens = mlp_forward(F, b1, b2, w3, b3, lane, feat, act);
-      const float rho = in ? dens * net.rho_scale : 0.0f;
-      const float yk = rho - comp;
-      const float tt = acc + yk;
-      comp = (tt - acc) - yk;
-      acc = tt;
+  unsigned long long n_samples = 0;
+
+  for (;;) {
+    unsigned tile = 0;
+    if (lane == 0) tile = atomicAdd(p.counts, 1u);
+    tile = __builtin_amdgcn_readfirstlane(tile);
+    if (tile >= n_tiles) break;
+    const int v = (int)(tile / per_view);
+    const int in_view = (int)(tile - (unsigned)v * per_view);
+    const int ti = in_view / tiles_j, tj = in_view - ti * tiles_j;
+    const int i = ti * 4 + (s >> 2);
+    const int j = tj * 4 + (s & 3);
+    const bool valid = i < p.res && j < p.res;
+
+    long k_lo = 1, k_hi = 0;
+    Ray r;
+    r.o[0] = r.o[1] = r.o[2] = 0.0;
+    r.d[0] = r.d[1] = r.d[2] = 0.0;
+    if (valid) {
+      r = make_ray(p, p.views[p.view_offset + v], i, j);
+      double t_in, t_out;
+      if (clip_ray(p, r, t_in, t_out)) {
+        double a = floor((t_in - p.smin) / ds_sur - 0.5) - 1.0;
+        double b = ceil((t_out - p.smin) / ds_sur - 0.5) + 1.0;
+        k_lo = a > 0.0 ? (long)a : 0;
+        k_hi = b < (double)(K - 1) ? (long)b : K - 1;
+      }
+    }
+    long wlo = k_lo, whi = k_hi;
+    // the union of the wave's sample ranges (empty ranges have lo > hi)
+    if (k_lo > k_hi) {
+      wlo = 0x7fffffffffffL;
+      whi = -1;
+    }
+#pragma unroll
+    for (int o = 1; o < 64; o <<= 1) {
+      wlo = min(wlo, (long)__shfl_xor(wlo, o, 64));
+      whi = max(whi, (long)__shfl_xor(whi, o, 64));
+    }
+    if (whi >= wlo) n_samples += (unsigned long long)(whi - wlo + 1) * 16ull;
+    float acc = 0.0f, comp = 0.0f;
+    const float d0 = (float)r.d[0], d1 = (float)r.d[1], d2 = (float)r.d[2];
+    for (long k0 = wlo; k0 <= whi; k0 += kChunk) {
+      const double sa = p.smin + ((double)k0 + 0.5) * ds_sur;
+      const float a0 = (float)(r.o[0] + r.d[0] * sa), a1 = (float)(r.o[1] + r.d[1] * sa),
+                  a2 = (float)(r.o[2] + r.d[2] * sa);
+      const int n = (int)min((long)kChunk, whi - k0 + 1);
+      // the ray's own samples of the chunk
+      const int lo = (int)max(min(k_lo - k0, (long)kChunk), 0l),
+                hi = (int)max(min(k_hi - k0, (long)kChunk), -1l);
+      for (int jj = 0; jj < n; ++jj) {
+        const float sj = (float)jj * dsf;
+        float x = fmaf(d0, sj, a0), y = fmaf(d1, sj, a1), z = fmaf(d2, sj, a2);
+        deform32(p.defs, p.n_defs, x, y, z);
+        float ux = 0.5f, uy = 0.5f, uz = 0.5f;
+        const bool in = sur_domain(net, x, y, z, ux, uy, uz) && jj >= lo && jj <= hi;
+        float feat[8];
+        encode_bf16(net.table_bf16, L.tab, tmask, levels, in ? ux : 0.5f, in ? uy : 0.5f,
+                    in ? uz : 0.5f, feat);
+        // an index the compiler takes as new in every step: it would otherwise
+        // keep the operands in 144 registers
+        int operand_lane = lane;
+        asm volatile("" : "+v"(operand_lane));
+        const float dens = mlp_density(L, b3, operand_lane, feat);
+        const float rho = in ? dens * net.rho_scale : 0.0f;
+        const float yk = rho - comp;
+        const float tt = acc + yk;
+        comp = (tt - acc) - yk;
+        acc = tt;
+      }
+    }
+    if (valid && g == 0) {
+      const double T = p.flat_field + ((double)acc * p.dm) * ds_sur;
+      store_pixel(p, v, i, j, T);
     }
   }
-  if (valid && g == 0) {
-    const double T = p.flat_field + ((double)acc * p.dm) * ds_sur;
-    store_pixel(p, v, i, j, T);
-  }
+  if (p.stats && lane == 0 && n_samples) atomicAdd(p.stats + ST_SAMPLES, n_samples);
 }
 
 // ---------------------------------------------------------------------------
@@ -744,9 +902,13 @@ int launch_sur_predict(const SurNet& net, const float* pts, int64_t n, float* ou
 
 int launch_sur_render(const SurNet& net, const MarchParams& p, double ds_sur, void* stream) {
   const long K = (long)std::ceil((p.smax - p.smin) / ds_sur);
-  const int tiles = (p.res + 3) / 4;
-  hipLaunchKernelGGL(sur_render_kernel, dim3(tiles * tiles, p.n_views), dim3(64), 0,
-                     (hipStream_t)stream, net, p, ds_sur, K);
+  const int64_t tiles = (int64_t)((p.res + 3) / 4) * ((p.res + 3) / 4) * p.n_views;
+  // tile numbers go past the last by one per wave
+  if (tiles > 0xf0000000ll || !p.counts) return (int)hipErrorInvalidValue;
+  const int64_t groups = (tiles + kSurMarchWaves - 1) / kSurMarchWaves;
+  hipLaunchKernelGGL(sur_render_kernel, dim3((unsigned)std::min<int64_t>(groups, kSurGroups)),
+                     dim3(64 * kSurMarchWaves), 0, (hipStream_t)stream, net, p, ds_sur, K,
+                     (unsigned)tiles);
   return (int)hipGetLastError();
 }
 
