@@ -2001,11 +2001,12 @@ struct xrp_surrogate {
   int64_t table_count = 0;  // of which tables
   DevBuf params, grads, m, v, tbf16, loss, pts, labels, scene_nodes, items, vals;
   DevBuf judge, counters;  // certified check: exact images, tile counters
+  DevBuf work;             // training: at most 33 MiB (sur_train_bytes)
   int adam_step = 0;
   bool packed = false;
   ~xrp_surrogate() {
     for (DevBuf* b : {&params, &grads, &m, &v, &tbf16, &loss, &pts, &labels, &scene_nodes,
-                      &items, &vals, &judge, &counters})
+                      &items, &vals, &judge, &counters, &work})
       b->release();
   }
 };
@@ -2210,11 +2211,12 @@ int xrp_surrogate_gradients(xrp_surrogate* s, const float* u_host, const float* 
     HIPCHK(s->labels.ensure((size_t)n * sizeof(float)));
     HIPCHK(hipMemcpy(s->pts.p, u_host, (size_t)n * 3 * sizeof(float), hipMemcpyHostToDevice));
     HIPCHK(hipMemcpy(s->labels.p, targets, (size_t)n * sizeof(float), hipMemcpyHostToDevice));
+    HIPCHK(s->work.ensure(sur_train_bytes(s->net, n)));
     HIPCHK(hipMemsetAsync(s->grads.p, 0, (size_t)s->count * sizeof(float), s->ctx->stream));
     HIPCHK(hipMemsetAsync(s->loss.p, 0, sizeof(double), s->ctx->stream));
     int e = launch_sur_train(s->net, (const float*)s->pts.p, (const float*)s->labels.p, n,
                              (float)(1.0 / (double)n), (float*)s->grads.p, (double*)s->loss.p,
-                             s->ctx->stream);
+                             s->work.p, s->ctx->stream);
     if (e) return fail(XRP_ERR_DEVICE, hipGetErrorString((hipError_t)e));
     HIPCHK(hipStreamSynchronize(s->ctx->stream));
     HIPCHK(hipMemcpy(grads_host, s->grads.p, (size_t)s->count * sizeof(float),
@@ -2242,6 +2244,7 @@ int xrp_surrogate_train(xrp_surrogate* s, const xrp_train_config* cfg, xrp_train
     const int64_t n = cfg->samples;
     HIPCHK(s->pts.ensure((size_t)n * 3 * sizeof(float)));
     HIPCHK(s->labels.ensure((size_t)n * sizeof(float)));
+    HIPCHK(s->work.ensure(sur_train_bytes(s->net, std::min<int64_t>(n, cfg->batch))));
     MarchParams scene;
     std::memset(&scene, 0, sizeof scene);
     scene.nodes = (const DevNode*)s->scene_nodes.p;
@@ -2265,7 +2268,7 @@ int xrp_surrogate_train(xrp_surrogate* s, const xrp_train_config* cfg, xrp_train
         HIPCHK(hipMemsetAsync(s->grads.p, 0, (size_t)s->count * sizeof(float), ctx->stream));
         e = launch_sur_train(s->net, (const float*)s->pts.p + 3 * b0,
                              (const float*)s->labels.p + b0, nb, (float)(1.0 / (double)nb),
-                             (float*)s->grads.p, (double*)s->loss.p, ctx->stream);
+                             (float*)s->grads.p, (double*)s->loss.p, s->work.p, ctx->stream);
         if (!e)
           e = launch_sur_adam((float*)s->params.p, (const float*)s->grads.p, (float*)s->m.p,
                               (float*)s->v.p, s->count, s->table_count, (float)cfg->lr_table,

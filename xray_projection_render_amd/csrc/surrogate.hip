@@ -115,12 +115,18 @@ __device__ __forceinline__ void encode_f32(const SurNet& net, int g, float ux, f
     const int l = lane_level(g, q);
     const int N = net.res[l];
     const LevelCell c = level_cell(N, tmask, level_dense(N, net.log2_table), ux, uy, uz);
+    // corners along x, mostly of one line, one after the other
+    float2 e[8];
+#pragma unroll
+    for (int j = 0; j < 8; ++j) {
+      const int k = (j >> 1) | ((j & 1) << 2);
+      e[k] = tab[(size_t)l * T + c.idx[k]];
+    }
     float f0 = 0.0f, f1 = 0.0f;
 #pragma unroll
     for (int k = 0; k < 8; ++k) {
-      const float2 e = tab[(size_t)l * T + c.idx[k]];
-      f0 = fmaf(c.w[k], e.x, f0);
-      f1 = fmaf(c.w[k], e.y, f1);
+      f0 = fmaf(c.w[k], e[k].x, f0);
+      f1 = fmaf(c.w[k], e[k].y, f1);
     }
     feat[2 * q] = f0;
     feat[2 * q + 1] = f1;
@@ -259,10 +265,48 @@ __global__ void sur_labels_kernel(SurNet net, MarchParams scene, uint64_t seed, 
 }
 
 // ---------------------------------------------------------------------------
-// Training step: forward, backward, gradient accumulation.
+// Training step: forward, backward, gradient accumulation, in three kernels.
+// Global memory takes 18 G FP32 adds/s wherever they land, and a step of n
+// samples makes 256 n for the tables, and one kernel made 6337 per wave for the
+// MLP.  So the first kernel only writes the gradients of the features, and each
+// workgroup its own sum of the MLP's gradients, which the second adds up; in the
+// third every slice of a table has a workgroup that owns it, meets all samples
+// and adds in LDS (three cycles a lane: small levels, all of whose corners are
+// in one slice, are shared out over parts of the samples as well).  65536
+// samples, 2^17-entry tables: 940 us -> 82 + 7 + 188 us; a whole training step
+// with 2^14, 2^17, 2^19 and 2^21 entries 0.96, 0.97, 1.02, 1.37 -> 0.24, 0.30,
+// 0.40, 0.84 ms, of 1000 samples 0.33, 0.35, 0.40, 0.79 -> 0.07, 0.09, 0.15,
+// 0.48.  Every workgroup meets all samples, so the gain goes with the number of
+// slices: beyond kSurSlicesMost (2^22 entries and up) the tables' adds stay in
+// global memory.
 // ---------------------------------------------------------------------------
 constexpr int kSurTrainWaves = 4;
-constexpr int kSurGroupsPerWave = 8;  // 128 samples per wave between flushes
+constexpr int kSurTrainGroups = 256;         // workgroups of a launch, at most
+constexpr uint32_t kSurSlice = 8192;         // entries of a slice: 64 KiB of LDS
+constexpr int kSurScatterWaves = 16;
+constexpr uint32_t kSurParts = 16;           // workgroups of a level, at least
+constexpr uint32_t kSurSlicesMost = 4096;
+constexpr int64_t kSurTrainChunk = 1 << 17;  // samples of a launch, at most
+
+// Entries that level l's cells reach.
+__host__ __device__ inline uint32_t sur_entries(const SurNet& net, int l) {
+  const uint64_t n1 = (uint64_t)net.res[l] + 1u, t = 1ull << net.log2_table;
+  // n1^3 <= t: the level is dense
+  return (uint32_t)(n1 <= 4096u && n1 * n1 * n1 <= t ? n1 * n1 * n1 : t);
+}
+// Slices of a level, and workgroups of each (each with a part of the samples).
+struct SurSlices {
+  uint32_t n, parts;
+};
+__host__ __device__ inline SurSlices sur_slices(const SurNet& net, int l) {
+  const uint32_t n = (sur_entries(net, l) + kSurSlice - 1) / kSurSlice;
+  return {n, n < kSurParts ? (kSurParts + n - 1) / n : 1u};
+}
+inline uint32_t sur_slices(const SurNet& net) {
+  uint32_t n = 0;
+  for (int l = 0; l < kSurLevels; ++l) n += sur_slices(net, l).n * sur_slices(net, l).parts;
+  return n;
+}
 
 struct SurWaveLds {
   short t1[64][16];  // h1 (post ReLU, bf16) [unit][sample]
@@ -278,10 +322,12 @@ __device__ __forceinline__ bf16x4 lds_row4(const short (*t)[16], int unit, int s
   return v;
 }
 
+// dx: the samples' feature gradients, [level][sample], or null (adds to the
+// tables' gradients in `grads`).  sums: kSurMlpParams of each workgroup.
 __global__ __launch_bounds__(256) void sur_train_kernel(SurNet net, const float* pts,
                                                         const float* labels, int64_t n,
-                                                        float inv_n, float* grads,
-                                                        double* loss_sum) {
+                                                        float inv_n, float* grads, float2* dx_out,
+                                                        float* sums, double* loss_sum) {
   __shared__ SurFwdLds F;
   __shared__ SurBwdLds B;
   __shared__ SurWaveLds WL[kSurTrainWaves];
@@ -289,6 +335,8 @@ __global__ __launch_bounds__(256) void sur_train_kernel(SurNet net, const float*
   const float* P = net.params;
   stage_fwd(F, P + off.W1, P + off.W2);
   stage_bwd(B, P + off.W1, P + off.W2);
+  __shared__ float sum[kSurMlpParams];
+  for (int e = threadIdx.x; e < kSurMlpParams; e += blockDim.x) sum[e] = 0.0f;
   __syncthreads();
 
   const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
@@ -315,11 +363,10 @@ __global__ __launch_bounds__(256) void sur_train_kernel(SurNet net, const float*
   for (int q = 0; q < 16; ++q) db1[q] = db2[q] = dw3[q] = 0.0f;
   float db3 = 0.0f, sq = 0.0f;
 
-  const int64_t wave_id = (int64_t)blockIdx.x * kSurTrainWaves + wave;
-  const int64_t first = wave_id * 16 * kSurGroupsPerWave;
-  for (int grp = 0; grp < kSurGroupsPerWave; ++grp) {
-    const int64_t k = first + (int64_t)grp * 16 + s;
-    if (first + (int64_t)grp * 16 >= n) break;  // wave-uniform
+  const int64_t step = (int64_t)gridDim.x * kSurTrainWaves * 16;
+  for (int64_t first = ((int64_t)blockIdx.x * kSurTrainWaves + wave) * 16; first < n;
+       first += step) {
+    const int64_t k = first + s;
     const bool ok = k < n;
     const float ux = ok ? pts[3 * k] : 0.5f, uy = ok ? pts[3 * k + 1] : 0.5f,
                 uz = ok ? pts[3 * k + 2] : 0.5f;
@@ -376,7 +423,11 @@ __global__ __launch_bounds__(256) void sur_train_kernel(SurNet net, const float*
       }
     }
     // hash table gradients (only real samples)
-    if (ok) {
+    if (ok && dx_out) {
+#pragma unroll
+      for (int q = 0; q < 4; ++q)
+        dx_out[(int64_t)lane_level(g, q) * n + k] = make_float2(dx[2 * q], dx[2 * q + 1]);
+    } else if (ok) {
 #pragma unroll
       for (int q = 0; q < 4; ++q) {
         const int l = lane_level(g, q);
@@ -415,51 +466,122 @@ __global__ __launch_bounds__(256) void sur_train_kernel(SurNet net, const float*
     __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "wavefront");
   }
 
-  // flush: weight tiles hold D[m = 4g+i][n = s] of each (mt, nt) tile
-  float* gW1 = grads + off.W1;
-  float* gW2 = grads + off.W2;
-#pragma unroll
-  for (int mt = 0; mt < 4; ++mt)
-#pragma unroll
-    for (int nt = 0; nt < 4; ++nt)
-#pragma unroll
-      for (int i = 0; i < 4; ++i)
-        atomicAdd(gW2 + (size_t)(16 * mt + 4 * g + i) * kSurHidden + 16 * nt + s,
-                  accW2[mt][nt][i]);
-#pragma unroll
-  for (int mt = 0; mt < 2; ++mt)
-#pragma unroll
-    for (int nt = 0; nt < 4; ++nt)
-#pragma unroll
-      for (int i = 0; i < 4; ++i)
-        atomicAdd(gW1 + (size_t)(16 * mt + 4 * g + i) * kSurHidden + 16 * nt + s,
-                  accW1[mt][nt][i]);
   // per-unit sums over the 16 samples (lanes of one group)
 #pragma unroll
-  for (int q = 0; q < 16; ++q) {
-    float a1 = db1[q], a2 = db2[q], a3 = dw3[q];
+  for (int q = 0; q < 16; ++q)
 #pragma unroll
     for (int o = 1; o < 16; o <<= 1) {
-      a1 += __shfl_xor(a1, o, 64);
-      a2 += __shfl_xor(a2, o, 64);
-      a3 += __shfl_xor(a3, o, 64);
+      db1[q] += __shfl_xor(db1[q], o, 64);
+      db2[q] += __shfl_xor(db2[q], o, 64);
+      dw3[q] += __shfl_xor(dw3[q], o, 64);
     }
-    if (s == 0) {
-      const int u = 16 * (q >> 2) + 4 * g + (q & 3);
-      atomicAdd(grads + off.b1 + u, a1);
-      atomicAdd(grads + off.b2 + u, a2);
-      atomicAdd(grads + off.w3 + u, a3);
-    }
-  }
-  float r3 = db3, rs = sq;
 #pragma unroll
   for (int o = 1; o < 64; o <<= 1) {
-    r3 += __shfl_xor(r3, o, 64);
-    rs += __shfl_xor(rs, o, 64);
+    db3 += __shfl_xor(db3, o, 64);
+    sq += __shfl_xor(sq, o, 64);
   }
-  if (lane == 0) {
-    atomicAdd(grads + off.b3, r3);
-    atomicAdd(loss_sum, (double)rs);
+  if (lane == 0) atomicAdd(loss_sum, (double)sq);
+  // the workgroup's sum, a wave after the other (adds in LDS by atomics take
+  // three cycles a lane); weight tiles hold D[m = 4g+i][n = s] of each (mt, nt)
+  float* gW2 = sum + (off.W2 - off.W1);
+  for (int w = 0; w < kSurTrainWaves; ++w) {
+    __syncthreads();
+    if (wave != w) continue;
+#pragma unroll
+    for (int nt = 0; nt < 4; ++nt)
+#pragma unroll
+      for (int i = 0; i < 4; ++i) {
+#pragma unroll
+        for (int mt = 0; mt < 4; ++mt)
+          gW2[(16 * mt + 4 * g + i) * kSurHidden + 16 * nt + s] += accW2[mt][nt][i];
+#pragma unroll
+        for (int mt = 0; mt < 2; ++mt)
+          sum[(16 * mt + 4 * g + i) * kSurHidden + 16 * nt + s] += accW1[mt][nt][i];
+      }
+    if (s == 0) {
+#pragma unroll
+      for (int q = 0; q < 16; ++q) {
+        const int u = 16 * (q >> 2) + 4 * g + (q & 3);
+        sum[off.b1 - off.W1 + u] += db1[q];
+        sum[off.b2 - off.W1 + u] += db2[q];
+        sum[off.w3 - off.W1 + u] += dw3[q];
+      }
+    }
+    if (lane == 0) sum[off.b3 - off.W1] += db3;
+  }
+  __syncthreads();
+  float* out = sums + (size_t)blockIdx.x * kSurMlpParams;
+  for (int e = threadIdx.x; e < kSurMlpParams; e += blockDim.x) out[e] = sum[e];
+}
+
+// grads[e] += the workgroups' sums: 64 parameters a workgroup, a wave per 16th
+// of the sums.
+__global__ __launch_bounds__(1024) void sur_sum_kernel(const float* sums, int groups,
+                                                       float* grads) {
+  __shared__ float part[16][64];
+  const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
+  const int e = blockIdx.x * 64 + lane;
+  float a = 0.0f;
+  if (e < kSurMlpParams)
+    for (int q = wave; q < groups; q += 16) a += sums[(size_t)q * kSurMlpParams + e];
+  part[wave][lane] = a;
+  __syncthreads();
+  if (wave == 0 && e < kSurMlpParams) {
+    for (int q = 1; q < 16; ++q) a += part[q][lane];
+    grads[e] += a;
+  }
+}
+
+// The tables' gradients: a slice of kSurSlice entries of a level per workgroup,
+// over all samples or a part of them.
+__global__ __launch_bounds__(64 * kSurScatterWaves) void sur_scatter_kernel(
+    SurNet net, const float* __restrict__ pts, const float2* __restrict__ dx, int64_t n,
+    float* grads) {
+  __shared__ float acc0[kSurSlice], acc1[kSurSlice];
+  // the workgroup's level, part and slice
+  int l = 0;
+  uint32_t b = blockIdx.x;
+  SurSlices sl = sur_slices(net, 0);
+  while (b >= sl.n * sl.parts) {
+    b -= sl.n * sl.parts;
+    sl = sur_slices(net, ++l);
+  }
+  const uint32_t part = b / sl.n, first = (b - part * sl.n) * kSurSlice;
+  const uint32_t count = min(sur_entries(net, l) - first, kSurSlice);
+  for (uint32_t e = threadIdx.x; e < count; e += blockDim.x) acc0[e] = acc1[e] = 0.0f;
+  __syncthreads();
+  const uint32_t tmask = (1u << net.log2_table) - 1u;
+  const int N = net.res[l];
+  const bool dense = level_dense(N, net.log2_table);
+  const float2* d = dx + (int64_t)l * n;
+  for (int64_t k = (int64_t)part * blockDim.x + threadIdx.x; k < n;
+       k += (int64_t)sl.parts * blockDim.x) {
+    const float2 t = d[k];
+    const LevelCell c =
+        level_cell(N, tmask, dense, pts[3 * k], pts[3 * k + 1], pts[3 * k + 2]);
+#pragma unroll
+    for (int q = 0; q < 8; ++q) {
+      const uint32_t at = c.idx[q] - first;
+      if (at < count) {
+        atomicAdd(acc0 + at, c.w[q] * t.x);
+        atomicAdd(acc1 + at, c.w[q] * t.y);
+      }
+    }
+  }
+  __syncthreads();
+  float2* g = (float2*)grads + (((size_t)l << net.log2_table) + first);
+  for (uint32_t e = threadIdx.x; e < count; e += blockDim.x) {
+    const float2 a = make_float2(acc0[e], acc1[e]);
+    if (a.x == 0.0f && a.y == 0.0f) continue;
+    if (sl.parts == 1) {
+      float2 v = g[e];
+      v.x += a.x;
+      v.y += a.y;
+      g[e] = v;
+    } else {
+      atomicAdd(&g[e].x, a.x);
+      atomicAdd(&g[e].y, a.y);
+    }
   }
 }
 
@@ -549,12 +671,6 @@ struct SurLevels {
   uint32_t y[4], z[4], first[4];
   bool dense[4], lds[4];
 };
-
-// Entries that level l's cells reach.
-__device__ __forceinline__ uint32_t sur_entries(const SurNet& net, int l) {
-  const uint32_t n1 = (uint32_t)net.res[l] + 1u;
-  return level_dense(net.res[l], net.log2_table) ? n1 * n1 * n1 : 1u << net.log2_table;
-}
 
 __device__ __forceinline__ SurLevels sur_levels(const SurNet& net, int g, int n_lds) {
   SurLevels L;
@@ -864,13 +980,34 @@ int launch_sur_labels(const SurNet& net, const MarchParams& scene, uint64_t seed
   return (int)hipGetLastError();
 }
 
+static int64_t sur_train_chunk(int64_t n) { return std::min(n, kSurTrainChunk); }
+
+size_t sur_train_bytes(const SurNet& net, int64_t n) {
+  const size_t sums = (size_t)kSurTrainGroups * kSurMlpParams * sizeof(float);
+  return sums + (sur_slices(net) <= kSurSlicesMost
+                     ? (size_t)sur_train_chunk(n) * kSurLevels * sizeof(float2)
+                     : 0);
+}
+
 int launch_sur_train(const SurNet& net, const float* pts, const float* labels, int64_t n,
-                     float inv_n, float* grads, double* loss_sum, void* stream) {
-  if (n <= 0) return 0;
-  const int64_t per_block = (int64_t)kSurTrainWaves * 16 * kSurGroupsPerWave;
-  hipLaunchKernelGGL(sur_train_kernel, dim3((unsigned)((n + per_block - 1) / per_block)),
-                     dim3(64 * kSurTrainWaves), 0, (hipStream_t)stream, net, pts, labels, n,
-                     inv_n, grads, loss_sum);
+                     float inv_n, float* grads, double* loss_sum, void* work, void* stream) {
+  const uint32_t slices = sur_slices(net);
+  float2* dx = slices <= kSurSlicesMost ? (float2*)work : nullptr;
+  float* sums = (float*)work + (dx ? (size_t)sur_train_chunk(n) * kSurLevels * 2 : 0);
+  hipStream_t s = (hipStream_t)stream;
+  for (int64_t at = 0; at < n; at += kSurTrainChunk) {
+    const int64_t c = std::min(n - at, kSurTrainChunk);
+    const int64_t waves = (c + 15) / 16;
+    const int groups =
+        (int)std::min<int64_t>((waves + kSurTrainWaves - 1) / kSurTrainWaves, kSurTrainGroups);
+    hipLaunchKernelGGL(sur_train_kernel, dim3(groups), dim3(64 * kSurTrainWaves), 0, s, net,
+                       pts + 3 * at, labels + at, c, inv_n, grads, dx, sums, loss_sum);
+    hipLaunchKernelGGL(sur_sum_kernel, dim3((kSurMlpParams + 63) / 64), dim3(1024), 0, s, sums,
+                       groups, grads + sur_table_floats(net.log2_table));
+    if (dx)
+      hipLaunchKernelGGL(sur_scatter_kernel, dim3(slices), dim3(64 * kSurScatterWaves), 0, s,
+                         net, pts + 3 * at, dx, c, grads);
+  }
   return (int)hipGetLastError();
 }
 

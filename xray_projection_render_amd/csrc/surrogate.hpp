@@ -46,9 +46,10 @@ __host__ __device__ inline size_t sur_param_count(int log2_table) {
 int launch_sur_labels(const SurNet& net, const MarchParams& scene, uint64_t seed,
                       int64_t n, float* pts, float* labels, void* stream);
 // Loss and gradients of a batch (grads accumulated, loss_sum += sum of
-// squared errors).  Points are u in [0,1]^3.
+// squared errors).  Points are u in [0,1]^3.  work: sur_train_bytes of n.
+size_t sur_train_bytes(const SurNet& net, int64_t n);
 int launch_sur_train(const SurNet& net, const float* pts, const float* labels, int64_t n,
-                     float inv_n, float* grads, double* loss_sum, void* stream);
+                     float inv_n, float* grads, double* loss_sum, void* work, void* stream);
 int launch_sur_adam(float* params, const float* grads, float* m, float* v, int64_t count,
                     int64_t table_count, float lr_table, float lr_mlp, float beta1,
                     float beta2, float eps, int step, void* stream);
