@@ -1002,6 +1002,25 @@ int plan_job(xrp_context* ctx, xrp_scene* sc, const RenderJob& job, LaunchPlan& 
     // FP32 anchor rounding (u*|G|) plus the FP32 step (4u * |B| * chunk*ds).
     mp.vguard = (float)(4.0 * (u * (N + 4.0 * L * 0.5 * N * 32.0 * job.ds) + 1e-9));
   }
+  // FP64 marches of a voxel root read its quad bricks (built on first use;
+  // for a launch without allocation, where they are there already), or the
+  // linear copy where the quads would pass 4 GiB or have no room
+  if (allow_voxel_kernel && s.root.kind == K_VOXEL && !vox_kernel &&
+      precision == XRP_PRECISION_FP64) {
+    mp.vlin = (const float*)vptr.front();
+    mp.vn[0] = s.root.nx;
+    mp.vn[1] = s.root.ny;
+    mp.vn[2] = s.root.nz;
+    mp.vbricks[0] = (s.root.nx + 3) / 4;
+    mp.vbricks[1] = (s.root.ny + 3) / 4;
+    mp.vbricks[2] = (s.root.nz + 3) / 4;
+    std::vector<void*> q;
+    if ((size_t)mp_bricks(s.root) * 64 < ((size_t)1 << 28) &&
+        upload_voxels(ctx, sc, q, SLOT_QUAD, no_alloc) == XRP_OK)
+      mp.vgrid = (const float*)q[q.size() - N_SLOTS + SLOT_QUAD];
+    else
+      (void)hipGetLastError();
+  }
   if (line.line) {
     mp.line = line.line;
     mp.line_cap = line.line_cap;

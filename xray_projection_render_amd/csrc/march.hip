@@ -50,6 +50,13 @@ namespace xrp {
 constexpr int march_tile_i(int) { return 32; }
 constexpr int march_tile_j(int) { return 2; }
 
+// Samples a visit of the FP64 march of a voxel root (march_ray.hpp
+// voxel_along64).  120 x 100 x 90 voxels, 12 x 256^2, hierarchical: 0.66 ms with
+// the general FP64 evaluator (a call a sample, eight loads through a generic
+// pointer), 0.51 in blocks of 4 from the linear copy, 0.33 from the quads (0.38
+// in blocks of 2, 0.34 of 3).
+constexpr int kVoxelBlock = 4;
+
 // Q: queue the FP64 re-evaluations per wave (always at B = 4).
 template <int PREC, int INTEG, int B, bool Q = false>
 __global__ __launch_bounds__(64) __attribute__((amdgpu_waves_per_eu(
@@ -411,7 +418,20 @@ int launch_march(const MarchParams& p, int precision, int integrator,
   const int tiles = ((p.res + ti - 1) / ti) * ((p.res + tj - 1) / tj);
   dim3 grid(tiles, p.n_views);
   hipStream_t s = (hipStream_t)stream;
-  if (precision == PREC_FP64) {
+  if (precision == PREC_FP64 && p.vlin) {
+    if (integrator == INT_HIERARCHICAL && p.vgrid)
+      hipLaunchKernelGGL((march_kernel<PREC_QUADS, INT_HIERARCHICAL, kVoxelBlock>), grid, block,
+                         0, s, p);
+    else if (integrator == INT_HIERARCHICAL)
+      hipLaunchKernelGGL((march_kernel<PREC_VOXEL, INT_HIERARCHICAL, kVoxelBlock>), grid, block,
+                         0, s, p);
+    else if (p.vgrid)
+      hipLaunchKernelGGL((march_kernel<PREC_QUADS, INT_SIMPLE, kVoxelBlock>), grid, block, 0, s,
+                         p);
+    else
+      hipLaunchKernelGGL((march_kernel<PREC_VOXEL, INT_SIMPLE, kVoxelBlock>), grid, block, 0, s,
+                         p);
+  } else if (precision == PREC_FP64) {
     if (integrator == INT_HIERARCHICAL)
       hipLaunchKernelGGL((march_kernel<PREC_FP64, INT_HIERARCHICAL, kBlock>), grid,
                          block, 0, s, p);

@@ -14,7 +14,11 @@ struct DevView {
 };
 
 enum Integrator : int32_t { INT_SIMPLE = 0, INT_HIERARCHICAL = 1 };
-enum Precision : int32_t { PREC_GUARDED = 0, PREC_FP64 = 1 };
+// PREC_VOXEL and PREC_QUADS: PREC_FP64 of a scene whose root is a voxel grid,
+// read from its linear copy (MarchParams::vlin) or its corner-quad bricks
+// (vgrid, VOX_BRICK4_QUAD).
+enum Precision : int32_t { PREC_GUARDED = 0, PREC_FP64 = 1, PREC_VOXEL = 2, PREC_QUADS = 3 };
+constexpr bool voxel_precision(int p) { return p == PREC_VOXEL || p == PREC_QUADS; }
 
 // Stat counters accumulated by the kernels (device, uint64 each).
 enum StatSlot {
@@ -74,7 +78,7 @@ struct MarchParams {
   double t[3];
   float vguard;            // grid units
   uint32_t vbytes;         // size of vgrid in bytes (buffer descriptor range)
-  const float* vlin;       // linear [z][x][y] copy (LDS staging source)
+  const float* vlin;       // linear [z][x][y] copy (LDS staging source; PREC_VOXEL)
   uint32_t vlin_bytes;
   // Output: 0 = float32 transmittance in out; 1 = the reference PNG's
   // 8-bit (gray, alpha) pair per pixel in out8 (main.go:481-498).

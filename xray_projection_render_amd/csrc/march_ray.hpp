@@ -33,6 +33,71 @@ struct RayCounts {
   unsigned long long samples = 0, reeval = 0, miss = 0, fine = 0, skipped = 0;
 };
 
+// FP64 densities at s[q] along the ray o + d s of a scene whose root is a
+// voxel grid, for the samples in `live` (0 for the others): voxel64's
+// operations (objects.go:789-855), B samples at a time so that their loads
+// overlap, with the grid's address and sizes from the launch parameters.
+// The gathers' lines bound it, so that the corner quads, two loads a cell in
+// place of eight, are read where the scene has them.
+template <int PREC, int B>
+__device__ __forceinline__ void voxel_along64(const MarchParams& p, const double (&o)[3],
+                                              const double (&d)[3], const double (&s)[B],
+                                              unsigned live, double (&rho)[B]) {
+  double x[B], y[B], z[B];
+#pragma unroll
+  for (int q = 0; q < B; ++q)
+    x[q] = o[0] + d[0] * s[q], y[q] = o[1] + d[1] * s[q], z[q] = o[2] + d[2] * s[q];
+  for (int k = 0; k < p.n_defs; ++k)
+#pragma unroll
+    for (int q = 0; q < B; ++q) deform64(p.defs + k, 1, x[q], y[q], z[q]);
+  const int nx = p.vn[0], ny = p.vn[1], nz = p.vn[2];
+  float v[B][8];
+  bool in[B];
+#pragma unroll
+  for (int q = 0; q < B; ++q) {
+    in[q] = ((live >> q) & 1u) && x[q] >= -1 && x[q] <= 1 && y[q] >= -1 && y[q] <= 1 &&
+            z[q] >= -1 && z[q] <= 1;
+    x[q] = (in[q] ? x[q] + 1 : 0.0) / 2 * (double)(nx - 1);
+    y[q] = (in[q] ? y[q] + 1 : 0.0) / 2 * (double)(ny - 1);
+    z[q] = (in[q] ? z[q] + 1 : 0.0) / 2 * (double)(nz - 1);
+    const int x0 = (int)x[q], y0 = (int)y[q], z0 = (int)z[q];  // all >= 0
+    const int x1 = min(x0 + 1, nx - 1);
+    x[q] -= (double)x0, y[q] -= (double)y0, z[q] -= (double)z0;
+    if constexpr (PREC == PREC_QUADS) {
+      // bricks (bz, bx, by) of voxels (lz, lx, ly), under 2^32 elements' bytes
+      const unsigned sx = (unsigned)p.vbricks[1] * 64u, sz = (unsigned)p.vbricks[0] * sx;
+      const unsigned yz = (unsigned)(z0 >> 2) * sz + (unsigned)(y0 >> 2) * 64u +
+                          (unsigned)(z0 & 3) * 16u + (unsigned)(y0 & 3);
+      const float4 e0 =
+          ((const float4*)p.vgrid)[yz + (unsigned)(x0 >> 2) * sx + (unsigned)(x0 & 3) * 4u];
+      const float4 e1 =
+          ((const float4*)p.vgrid)[yz + (unsigned)(x1 >> 2) * sx + (unsigned)(x1 & 3) * 4u];
+      // v[x][y][z]; the upper y and z are clamped in the copy
+      v[q][0] = e0.x, v[q][1] = e0.y, v[q][2] = e0.z, v[q][3] = e0.w;
+      v[q][4] = e1.x, v[q][5] = e1.y, v[q][6] = e1.z, v[q][7] = e1.w;
+    } else {
+      const int y1 = min(y0 + 1, ny - 1), z1 = min(z0 + 1, nz - 1);
+      const size_t a[4] = {((size_t)z0 * nx + x0) * ny, ((size_t)z1 * nx + x0) * ny,
+                           ((size_t)z0 * nx + x1) * ny, ((size_t)z1 * nx + x1) * ny};
+#pragma unroll
+      for (int c = 0; c < 4; ++c) {
+        v[q][4 * (c >> 1) + (c & 1)] = p.vlin[a[c] + y0];
+        v[q][4 * (c >> 1) + 2 + (c & 1)] = p.vlin[a[c] + y1];
+      }
+    }
+  }
+#pragma unroll
+  for (int q = 0; q < B; ++q) {
+    const double wx = x[q], wy = y[q], wz = z[q];
+    const double v00 = (double)v[q][0] * (1 - wz) + (double)v[q][1] * wz;
+    const double v01 = (double)v[q][2] * (1 - wz) + (double)v[q][3] * wz;
+    const double v10 = (double)v[q][4] * (1 - wz) + (double)v[q][5] * wz;
+    const double v11 = (double)v[q][6] * (1 - wz) + (double)v[q][7] * wz;
+    const double v0 = v00 * (1 - wy) + v01 * wy, v1 = v10 * (1 - wy) + v11 * wy;
+    rho[q] = in[q] ? v0 * (1 - wx) + v1 * wx : 0.0;
+  }
+}
+
 // First and last sample index of a ray's clipped segment (main.go:144-154;
 // s_k = s_table[k], s_{k+1} = s_k + ds).  Empty when k_hi < k_lo.
 __device__ __forceinline__ void clip_range(const MarchParams& p, double t_in, double t_out,
@@ -124,6 +189,39 @@ __device__ __forceinline__ double march_T_simple64(const MarchParams& p, int v, 
         double z = r.o[2] + r.d[2] * s;
         T += (density64(p, x, y, z) * p.dm) * ds;
         s += ds;
+      }
+      rc.samples += (unsigned long long)(k_hi - k_lo + 1);
+    }
+  }
+  return T;
+}
+
+// The same of a voxel root, B samples at a time.
+template <int PREC, int B>
+__device__ __forceinline__ double march_T_simple_voxel(const MarchParams& p, int v, int i, int j,
+                                                       RayCounts& rc) {
+  double T = p.flat_field;
+  Ray r = make_ray(p, p.views[p.view_offset + v], i, j);
+  double t_in, t_out;
+  if (clip_ray(p, r, t_in, t_out)) {
+    int k_lo, k_hi;
+    clip_range(p, t_in, t_out, k_lo, k_hi);
+    if (k_lo <= k_hi) {
+      const double ds = p.ds;
+      double s = p.s_table[k_lo];
+      for (int k = k_lo; k <= k_hi; k += B) {
+        double sq[B], rho[B];
+        unsigned live = 0;
+#pragma unroll
+        for (int q = 0; q < B; ++q) {
+          sq[q] = s;
+          if (k + q <= k_hi) live |= 1u << q;
+          s += ds;
+        }
+        voxel_along64<PREC, B>(p, r.o, r.d, sq, live, rho);
+#pragma unroll
+        for (int q = 0; q < B; ++q)
+          if ((live >> q) & 1u) T += (rho[q] * p.dm) * ds;
       }
       rc.samples += (unsigned long long)(k_hi - k_lo + 1);
     }
@@ -538,7 +636,9 @@ __device__ __forceinline__ void eval_along(const MarchParams& p, const double (&
                                            unsigned& amb, float* dist = nullptr,
                                            bool* last_amb = nullptr) {
   amb = 0;
-  if constexpr (PREC == PREC_FP64) {
+  if constexpr (voxel_precision(PREC)) {
+    voxel_along64<PREC, B>(p, o, d, s, live, rho);
+  } else if constexpr (PREC == PREC_FP64) {
 #pragma unroll
     for (int q = 0; q < B; ++q)
       rho[q] = ((live >> q) & 1u)
@@ -880,8 +980,12 @@ __device__ __forceinline__ double march_T(const MarchParams& p, int v, int i, in
                                           RayCounts& rc) {
   Cull cl;
   if constexpr (PREC == PREC_GUARDED) cl = wave_cull<QW>(p, v, i, j, valid);
-  if constexpr (INTEG == INT_HIERARCHICAL) {
+  if constexpr (INTEG == INT_HIERARCHICAL && voxel_precision(PREC)) {
+    return march_T_hier<PREC, QW, false, B, B>(p, v, i, j, valid, rc, cl);
+  } else if constexpr (INTEG == INT_HIERARCHICAL) {
     return march_T_hier<PREC, QW>(p, v, i, j, valid, rc, cl);
+  } else if constexpr (voxel_precision(PREC)) {
+    return valid ? march_T_simple_voxel<PREC, B>(p, v, i, j, rc) : 0.0;
   } else if constexpr (PREC == PREC_FP64) {
     return valid ? march_T_simple64(p, v, i, j, rc) : 0.0;
   } else if constexpr (DEFER) {
