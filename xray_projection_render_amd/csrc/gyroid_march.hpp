@@ -22,9 +22,9 @@
 // samples within reach of either end have that end's density, which leaves
 // about one to evaluate where the walk took four or five visits.
 //
-// Sheared 6^3 gyroid cells against the general march: 16 x 512^2 rays of
-// 1731 samples, simple, 1.60 -> 0.61 ms; 24 x 1024^2, hierarchical, 17.0 ->
-// 5.1 ms (first pass 12.8 -> 3.4, the FP64 passes 4.0 -> 1.6).
+// Sheared 6^3 gyroid cells against the general march: 16 x 512^2 rays at step
+// 0.001, simple, 1.60 -> 0.54 ms; 24 x 1024^2, hierarchical, 17.0 -> 3.75 ms
+// (first pass 12.8 -> 3.15, the FP64 passes 4.0 -> 0.54).
 //
 // Sums: every term is (rho * dm) * ds of one density value, so T is a number
 // of equal additions in a fixed order; the marches count and add at the end
@@ -50,9 +50,9 @@ struct GyroScene {
   float b0, b1, b2, b3, b4, b5, gb;  // the box and its band
   float cx, cy, cz, rv, rv_lo;       // centre, periods per length (two floats)
   float th, band;                    // level and band
-  float two_M, inv_M, e1, e3, inv;   // reach: 2M, 1/M, slope error (and 3 times), 1/scale
-  float per, far, first;             // samples per unit of box distance, of reach along
-                                     // the ray, and of | |g| - th | (1 / |grad g|)
+  float two_M, e1, e3, inv;          // reach: 2M, slope error (and 3 times), 1/scale
+  float per, far, first;             // samples per unit of box distance, of reach times M,
+                                     // and of | |g| - th | (1 / |grad g|)
   float A, k, Ak, sx, sy, sz, ax, ay, az;  // GYRO_TANH
 };
 
@@ -64,10 +64,10 @@ __device__ __forceinline__ GyroScene gyro_scene(const MarchParams& p, float per)
   s.gb = t.g[1];
   s.cx = g.f[0], s.cy = g.f[1], s.cz = g.f[2], s.rv = g.f[6], s.rv_lo = g.f[7];
   s.th = g.f[4], s.band = p.gyro_band;
-  s.two_M = 2.0f * g.g[6], s.inv_M = g.g[1], s.e1 = g.g[7], s.e3 = 3.0f * g.g[7];
+  s.two_M = 2.0f * g.g[6], s.e1 = g.g[7], s.e3 = 3.0f * g.g[7];
   s.inv = g.g[3];
   // the reach keeps eval_block.hpp's 1e-4 in hand
-  s.per = per, s.far = g.g[5] * per * (1.0f - 1e-4f), s.first = g.g[4] * per;
+  s.per = per, s.far = g.g[1] * g.g[5] * per * (1.0f - 1e-4f), s.first = g.g[4] * per;
   if constexpr (DEF == GYRO_TANH) {
     const DevDeform& f = p.defs[0];
     s.A = f.f[0], s.k = f.f[1], s.Ak = f.f[0] * f.f[1];
@@ -95,18 +95,22 @@ __device__ __forceinline__ void gyro_phase(float x, float c, const GyroScene& g,
   co = __builtin_amdgcn_cosf(r);
 }
 
-// Reach to a level at distance c of |g| (less its band), the slope along the
-// ray towards it at least -as and at most as in size as = |slope|: moving
+// Reach, times M, to a level at distance c of |g| (less its band) along a ray
+// whose slope towards it is as = |slope| in size, off by at most e1: moving
 // towards it, and away from it.  Towards: the root of c - (as + e1) s -
-// M s^2 / 2, 2c / (q + as + e1), q = sqrt((as + e1)^2 + 2 M c).  Away: that of
-// c + (as - e1) s - M s^2 / 2, (as - e1 + q') / M, whose q' = sqrt((as -
-// e1)^2 + 2 M c) is at least q - 2 e1: one root serves both.
+// M s^2 / 2, (q - as - e1) / M with q = sqrt((as + e1)^2 + 2 M c).  Away: that
+// of c + (as - e1) s - M s^2 / 2, (q' + as - e1) / M, whose q' = sqrt((as -
+// e1)^2 + 2 M c) is at least q - 2 e1: one root serves both.  1e-6 q covers
+// the rounding of the root and, where they cancel, of the difference: a loss of
+// 1e-6 of slope over curvature, 1e-4 of a fine step of 1e-4 on cells of 1/6.
+// (2 c / (q + as + e1) does not cancel but divides: simple first pass 559 against
+// 499 us, hierarchical 3.25 against 3.15 ms.)
 __device__ __forceinline__ void gyro_reach(const GyroScene& g, float c, float as, float& to,
                                            float& away) {
   const float b = as + g.e1;
-  const float q = b + __builtin_amdgcn_sqrtf(fmaf(b, b, g.two_M * c));
-  to = (c + c) * __builtin_amdgcn_rcpf(q);
-  away = (q - (g.e3 + g.e1)) * g.inv_M;  // q holds as + e1 too
+  const float q = __builtin_amdgcn_sqrtf(fmaf(b, b, g.two_M * c)) * (1.0f - 1e-6f);
+  to = q - b;
+  away = q + (as - g.e3);
 }
 
 template <int DEF>
