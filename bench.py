@@ -457,17 +457,18 @@ def measured_counter(name: str, kernel: str, workload: str):
 C5_WORKLOAD = "gyroid6_tanh_256x1024"
 
 
-def march_kernel_name(st: dict, integrator: str = "simple") -> str:
-    """The guarded march's dominant kernel as the render ran it: samples per
-    node visit, and the first pass of the two-pass form (whose other
-    launches are timed with it in kernel_ms)."""
-    if integrator != "simple":
-        if st.get("two_pass"):
-            return f"march_hier_try_kernel<{st['block']},2>"
-        return "march_kernel<PREC_GUARDED,INT_HIERARCHICAL>"
-    if st.get("two_pass"):
-        return f"march_try_kernel<{st['block']}>"
-    return f"march_kernel<PREC_GUARDED,INT_SIMPLE,{st['block']}>"
+def march_kernel_name(st: dict, integrator: str = "simple", scene: str = "gyroid") -> str:
+    """The guarded march's dominant kernel as the render ran it; launches
+    after a first pass are timed with it in kernel_ms.  The CSG scene and the
+    strut lattice take the interval march (a collection, a tessellation), the
+    gyroid lattice the gyroid march under a tanh displacement."""
+    two, hier = st.get("two_pass"), integrator != "simple"
+    if scene == "gyroid":
+        if two:
+            return "gyro_hier_try_kernel<1>" if hier else "gyro_try_kernel<1>"
+        return f"gyro_kernel<1,{int(hier)},false>"
+    kind = 1 if scene == "csg" else 2
+    return f"line_try_kernel<{kind}>" if two else f"line_kernel<{int(hier)},false,{kind}>"
 
 
 def bench_c5(args) -> int:
@@ -742,8 +743,8 @@ def main() -> int:
         roof["kernel"] = "march_kernel<%s,%s>" % (
             "PREC_FP64" if prec == "fp64" else "PREC_GUARDED",
             "INT_SIMPLE" if w.integrator == "simple" else "INT_HIERARCHICAL")
-        if st.get("block"):
-            roof["kernel"] = march_kernel_name(st, w.integrator)
+        if prec != "fp64" and w.name in ("csg", "lattice", "gyroid"):
+            roof["kernel"] = march_kernel_name(st, w.integrator, w.name)
     roof["skipped_samples"] = st.get("skipped_samples", 0)
     if roof["bound"] == "hbm":
         # the gathers mostly hit L2: also state them against the measured L2

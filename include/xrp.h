@@ -124,21 +124,25 @@ typedef struct {
   double kernel_ms;        /* device time of the render kernels */
   double position_error;   /* FP32 object-space position error bound used */
   int32_t precision_used;  /* xrp_precision actually run */
-  int32_t block;           /* samples per node visit of the guarded simple march
-                              (1, 2 or 4), or coarse samples per node visit of the
-                              two-pass hierarchical march's first pass; 0 for the
-                              other kernels */
+  int32_t block;           /* samples per node visit that the general guarded simple
+                              march takes for the scene (1, 2 or 4), or coarse
+                              samples per node visit of the two-pass hierarchical
+                              march's first pass; 0 for the other kernels */
   uint64_t staged_chunks;   /* voxel kernel: sample chunks served from LDS */
   uint64_t staged_voxels;   /* voxel kernel: voxels copied into LDS */
   uint64_t fallback_chunks; /* voxel kernel: chunks gathered from global memory */
   uint64_t skipped_samples; /* guarded marches: (coarse) samples whose density was settled
                                without evaluation, from the safe radius (distance to
                                the nearest boundary, less every FP32 error) of an
-                               evaluated sample before them; under audit each is
-                               also evaluated in FP64 and compared */
+                               evaluated sample before (or, fine samples of a
+                               gyroid lattice, after) them, or from the run of
+                               indices a convex primitive holds; under audit each
+                               is also evaluated in FP64 and compared */
   uint64_t redo_rays;       /* two-pass march: rays marched again (more guard-band
                                samples than a deferral slot holds, no slot free, or,
-                               hierarchical, an FP32 guess that was not exact) */
+                               hierarchical, an FP32 guess that was not exact; of
+                               straight rays through convex primitives: evaluated
+                               in FP64 throughout) */
   uint64_t deferred_rays;   /* two-pass march: rays whose guard-band samples were
                                re-evaluated (hierarchical: checked) in FP64 after
                                the march */
