@@ -457,16 +457,17 @@ def measured_counter(name: str, kernel: str, workload: str):
 C5_WORKLOAD = "gyroid6_tanh_256x1024"
 
 
-def march_kernel_name(st: dict, integrator: str = "simple", scene: str = "gyroid") -> str:
+def march_kernel_name(st: dict, integrator: str = "simple", scene: str = "gyroid",
+                      sheared: bool = True) -> str:
     """The guarded march's dominant kernel as the render ran it; launches
     after a first pass are timed with it in kernel_ms.  The CSG scene and the
     strut lattice take the interval march (a collection, a tessellation), the
-    gyroid lattice the gyroid march under a tanh displacement."""
+    gyroid lattice the gyroid march (0: undeformed, 1: a tanh displacement)."""
     two, hier = st.get("two_pass"), integrator != "simple"
     if scene == "gyroid":
         if two:
-            return "gyro_hier_try_kernel<1>" if hier else "gyro_try_kernel<1>"
-        return f"gyro_kernel<1,{int(hier)},false>"
+            return f"gyro_{'hier_' if hier else ''}try_kernel<{int(sheared)}>"
+        return f"gyro_kernel<{int(sheared)},{int(hier)},false>"
     kind = 1 if scene == "csg" else 2
     return f"line_try_kernel<{kind}>" if two else f"line_kernel<{int(hier)},false,{kind}>"
 
@@ -744,7 +745,7 @@ def main() -> int:
             "PREC_FP64" if prec == "fp64" else "PREC_GUARDED",
             "INT_SIMPLE" if w.integrator == "simple" else "INT_HIERARCHICAL")
         if prec != "fp64" and w.name in ("csg", "lattice", "gyroid"):
-            roof["kernel"] = march_kernel_name(st, w.integrator, w.name)
+            roof["kernel"] = march_kernel_name(st, w.integrator, w.name, bool(w.deformation))
     roof["skipped_samples"] = st.get("skipped_samples", 0)
     if roof["bound"] == "hbm":
         # the gathers mostly hit L2: also state them against the measured L2
