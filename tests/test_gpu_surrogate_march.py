@@ -65,10 +65,16 @@ def test_march_is_its_predictions(ctx, log2_table, n_min, n_max):
     p, at = np.concatenate(pts), np.concatenate(where)
     u = (p - w.obj["uc"]["xmin"]) / (w.obj["uc"]["xmax"] - w.obj["uc"]["xmin"])
     dens = sur.predict((u - np.floor(u)).astype(np.float32)).astype(np.float64)
-    sur.close()
     edge = (np.abs(p) >= 0.5 - EDGE).any(axis=1)
     T, E = (np.bincount(at[m], weights=dens[m] * ds, minlength=2 * res * res)
             .reshape(2, res, res) for m in (~edge, edge))
+    # two views of 48 x 48 tiles go to resident workgroups, one does not: the
+    # same bits
+    both, _ = sur.render(angles, 190, 0.5 * ds, ds, 0.0)
+    for v in range(2):
+        one, _ = sur.render(angles[v:v + 1], 190, 0.5 * ds, ds, 0.0)
+        assert np.array_equal(one[0], both[v])
+    sur.close()
     err = np.minimum(np.abs(img - np.exp(-T)), np.abs(img - np.exp(-(T + E))))
     print(f"{int(edge.sum())} samples at the bounds", flush=True)
     print(f"2^{log2_table}: max {err.max():.2e} mean {err.mean():.2e}", flush=True)

@@ -17,6 +17,7 @@
 
 #include <algorithm>
 #include <cmath>
+#include <type_traits>
 
 #include "eval_device.hpp"
 #include "march.hpp"
@@ -656,9 +657,11 @@ __device__ __forceinline__ bool sur_domain(const SurNet& net, float x, float y, 
 // The march's operands in LDS: the weights' and, per unit tile and lane group,
 // the four biases (of both layers) and output weights that group's lanes use.
 constexpr uint32_t kSurLdsEntries = 37600;  // 147 KiB
-struct SurMarchLds {
+struct SurMlpLds {
   SurFwdLds F;
   f32x4 b1[4][4], b2[4][4], w3[4][4];
+};
+struct SurMarchLds : SurMlpLds {
   uint32_t tab[kSurLdsEntries];  // tables of the first levels, as many as fit
 };
 static_assert(sizeof(SurMarchLds) <= 160 * 1024, "one workgroup a CU");
@@ -693,6 +696,7 @@ __device__ __forceinline__ SurLevels sur_levels(const SurNet& net, int g, int n_
 
 // The lane's features at u in [0, 1]^3 from the packed BF16 tables: all 32
 // gathers first, then the sums, whose terms and order are encode_f32's.
+template <bool LDS>
 __device__ __forceinline__ void encode_bf16(const uint32_t* __restrict__ tab,
                                             const uint32_t* lds_tab, uint32_t tmask,
                                             const SurLevels& L, float ux, float uy, float uz,
@@ -714,7 +718,7 @@ __device__ __forceinline__ void encode_bf16(const uint32_t* __restrict__ tab,
                      cz = z + (k & 1) * L.z[q];
       at[k] = L.first[q] + (L.dense[q] ? cx + cy + cz : (cx ^ cy ^ cz) & tmask);
     }
-    if (L.lds[q]) {
+    if (LDS && L.lds[q]) {
 #pragma unroll
       for (int k = 0; k < 8; ++k) e[q][k] = lds_tab[at[k]];
     } else {
@@ -744,7 +748,7 @@ __device__ __forceinline__ void encode_bf16(const uint32_t* __restrict__ tab,
 }
 
 // mlp_forward with its constants in LDS and no activations kept.
-__device__ __forceinline__ float mlp_density(const SurMarchLds& L, float b3, int lane,
+__device__ __forceinline__ float mlp_density(const SurMlpLds& L, float b3, int lane,
                                              const float (&feat)[8]) {
   const int g = lane >> 4;
   const bf16x4 x0 = f2bf4(feat[0], feat[1], feat[2], feat[3]);
@@ -774,7 +778,7 @@ __device__ __forceinline__ float mlp_density(const SurMarchLds& L, float b3, int
   return 1.0f / (1.0f + expf(-(part + b3)));
 }
 
-// One workgroup a CU, which stays for the launch: it stages the weights and
+// RESIDENT: one workgroup a CU, which stays for the launch: it stages the weights and
 // tables once, and its waves take tiles (16 rays, 4x4 pixels) from the counter
 // p.counts until none is left.
 //
@@ -790,12 +794,21 @@ __device__ __forceinline__ float mlp_density(const SurMarchLds& L, float b3, int
 // One 8-byte load for an aligned pair of corners: 2.58 ms.
 constexpr int kSurMarchWaves = 8;
 constexpr int kSurGroups = 256;
+// RESIDENT = false, for launches of fewer tiles than kSurResidentLeast: a
+// one-wave workgroup per tile, which keeps the operands in registers.  Such a
+// launch lasts as long as one wave's chain of steps, which the LDS reads
+// lengthen: 2^17-entry tables, 400, 2025, 3249, 4096 (one view, four views) and
+// 16384 tiles 0.45, 0.48, 0.69, 1.28, 1.55 and 2.51 ms, resident 0.93, 0.92,
+// 1.20, 1.26, 1.12 and 2.05 ms.
+constexpr unsigned kSurResidentLeast = 4096;
 
-__global__ __launch_bounds__(64 * kSurMarchWaves)
+template <bool RESIDENT>
+__global__ __launch_bounds__(RESIDENT ? 64 * kSurMarchWaves : 64)
     __attribute__((amdgpu_waves_per_eu(2))) void sur_render_kernel(SurNet net, MarchParams p,
                                                                    double ds_sur, long K,
                                                                    unsigned n_tiles) {
-  __shared__ SurMarchLds L;
+  __shared__ std::conditional_t<RESIDENT, SurMarchLds, SurMlpLds> L;
+  const uint32_t* lds_tab = nullptr;
   const SurOffsets off = sur_offsets(net.log2_table);
   const float* P = net.params;
   stage_fwd(L.F, P + off.W1, P + off.W2);
@@ -805,12 +818,15 @@ __global__ __launch_bounds__(64 * kSurMarchWaves)
     ((float*)L.w3)[threadIdx.x] = P[off.w3 + threadIdx.x];
   }
   int n_lds = 0;
-  for (uint32_t at = 0; n_lds < kSurLevels; ++n_lds) {
-    const uint32_t n = sur_entries(net, n_lds);
-    if (n > kSurLdsEntries - at) break;
-    const uint32_t* t = net.table_bf16 + ((size_t)n_lds << net.log2_table);
-    for (uint32_t e = threadIdx.x; e < n; e += blockDim.x) L.tab[at + e] = t[e];
-    at += n;
+  if constexpr (RESIDENT) {
+    lds_tab = L.tab;
+    for (uint32_t at = 0; n_lds < kSurLevels; ++n_lds) {
+      const uint32_t n = sur_entries(net, n_lds);
+      if (n > kSurLdsEntries - at) break;
+      const uint32_t* t = net.table_bf16 + ((size_t)n_lds << net.log2_table);
+      for (uint32_t e = threadIdx.x; e < n; e += blockDim.x) L.tab[at + e] = t[e];
+      at += n;
+    }
   }
   __syncthreads();
   const float b3 = P[off.b3];
@@ -823,11 +839,13 @@ __global__ __launch_bounds__(64 * kSurMarchWaves)
   const float dsf = (float)ds_sur;
   unsigned long long n_samples = 0;
 
-  for (;;) {
-    unsigned tile = 0;
-    if (lane == 0) tile = atomicAdd(p.counts, 1u);
-    tile = __builtin_amdgcn_readfirstlane(tile);
-    if (tile >= n_tiles) break;
+  for (bool more = true; more; more = RESIDENT) {
+    unsigned tile = blockIdx.x;
+    if constexpr (RESIDENT) {
+      if (lane == 0) tile = atomicAdd(p.counts, 1u);
+      tile = __builtin_amdgcn_readfirstlane(tile);
+      if (tile >= n_tiles) break;
+    }
     const int v = (int)(tile / per_view);
     const int in_view = (int)(tile - (unsigned)v * per_view);
     const int ti = in_view / tiles_j, tj = in_view - ti * tiles_j;
@@ -878,12 +896,12 @@ __global__ __launch_bounds__(64 * kSurMarchWaves)
         float ux = 0.5f, uy = 0.5f, uz = 0.5f;
         const bool in = sur_domain(net, x, y, z, ux, uy, uz) && jj >= lo && jj <= hi;
         float feat[8];
-        encode_bf16(net.table_bf16, L.tab, tmask, levels, in ? ux : 0.5f, in ? uy : 0.5f,
+        encode_bf16<RESIDENT>(net.table_bf16, lds_tab, tmask, levels, in ? ux : 0.5f, in ? uy : 0.5f,
                     in ? uz : 0.5f, feat);
         // an index the compiler takes as new in every step: it would otherwise
         // keep the operands in 144 registers
         int operand_lane = lane;
-        asm volatile("" : "+v"(operand_lane));
+        if constexpr (RESIDENT) asm volatile("" : "+v"(operand_lane));
         const float dens = mlp_density(L, b3, operand_lane, feat);
         const float rho = in ? dens * net.rho_scale : 0.0f;
         const float yk = rho - comp;
@@ -1042,10 +1060,12 @@ int launch_sur_render(const SurNet& net, const MarchParams& p, double ds_sur, vo
   const int64_t tiles = (int64_t)((p.res + 3) / 4) * ((p.res + 3) / 4) * p.n_views;
   // tile numbers go past the last by one per wave
   if (tiles > 0xf0000000ll || !p.counts) return (int)hipErrorInvalidValue;
-  const int64_t groups = (tiles + kSurMarchWaves - 1) / kSurMarchWaves;
-  hipLaunchKernelGGL(sur_render_kernel, dim3((unsigned)std::min<int64_t>(groups, kSurGroups)),
-                     dim3(64 * kSurMarchWaves), 0, (hipStream_t)stream, net, p, ds_sur, K,
-                     (unsigned)tiles);
+  if (tiles < kSurResidentLeast)
+    hipLaunchKernelGGL((sur_render_kernel<false>), dim3((unsigned)tiles), dim3(64), 0,
+                       (hipStream_t)stream, net, p, ds_sur, K, (unsigned)tiles);
+  else
+    hipLaunchKernelGGL((sur_render_kernel<true>), dim3(kSurGroups), dim3(64 * kSurMarchWaves), 0,
+                       (hipStream_t)stream, net, p, ds_sur, K, (unsigned)tiles);
   return (int)hipGetLastError();
 }
 
