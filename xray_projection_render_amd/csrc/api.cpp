@@ -808,16 +808,18 @@ int refresh_volume(xrp_context* ctx, xrp_scene* sc, const float* volume) {
 // by no more, over all of the box, than the FP32 rounding of a coordinate.
 //
 // mp.gyro_band, the error bound of the march's FP32 g (u = 2^-24): a
-// coordinate is off by delta from the position, u (bounds + |centre|) from
-// the subtraction of the centre and u bounds from the cells' sides; the
-// phase, reduced by one fma, by pi u twice.  |grad g| <= 1.77 (compute_guards)
-// over three coordinates so off: 1.77 sqrt(3) < 3.07 times that; the hardware
-// sine and cosine enter three products of two; 16 u for the products, the
-// sums and the level.  5 % in hand for the second-order terms with the
-// hierarchical integrator, whose fine samples lie at surfaces (a twelfth of
-// the general march's band: check and redo passes of 24 x 1024^2 rays 4.0 ->
-// 1.6 ms); four times the bound, as in compute_guards, with the simple one,
-// which has few samples in the band (resolve pass of 16 x 512^2: 36 us).
+// coordinate is off by delta from the position, u |centre| from the centre's
+// own rounding, u (bounds + |centre|) from its subtraction and u bounds from
+// the cells' sides; the phase, reduced by one fma, by pi u twice.  |grad g| <=
+// 1.77 (compute_guards) over three coordinates so off: 1.77 sqrt(3) < 3.07
+// times that; the hardware sine and cosine enter three products of two; 16 u
+// for the products, the sums and the level.  5 % in hand for the second-order
+// terms with the hierarchical integrator, whose fine samples lie at surfaces (a
+// twelfth of the general march's band: check and redo passes of 24 x 1024^2
+// rays 4.0 -> 1.6 ms).  With the simple one four times the bound, as in
+// compute_guards: few samples are in the band either way (resolve pass of 16 x
+// 512^2 36 us), and the tests of the deferral lists (tests/test_gpu_two_pass.py)
+// need rays with several of them: at 1.05, 32 rays of 8192 had one and none two.
 int gyroid_plan(const xrp::Scene& s, const std::vector<xrp::DevNode>& nodes, double delta,
                 bool simple, xrp::MarchParams& mp) {
   using namespace xrp;
@@ -840,7 +842,7 @@ int gyroid_plan(const xrp::Scene& s, const std::vector<xrp::DevNode>& nodes, dou
   double cm = 0.0;
   for (int k = 0; k < 3; ++k) cm = std::max(cm, std::fabs(g.d[k]));
   const double u = 1.0 / 16777216.0;
-  const double eq = (delta + u * (2.0 * bb + cm)) / g.d[3] + 2.0 * M_PI * u;
+  const double eq = (delta + u * (2.0 * bb + 2.0 * cm)) / g.d[3] + 2.0 * M_PI * u;
   const double kappa = simple ? 4.0 : 1.05;
   mp.gyro_band = (float)(kappa * (3.07 * eq + 6.0 * kHwSinCosErr + 16.0 * u));
   mp.gyro_tanh = s.ddefs.size() == 1 && s.ddefs[0].kind == D_TANH ? 1 : 0;
