@@ -2434,8 +2434,8 @@ int xrp_surrogate_render_device(xrp_surrogate* s, const xrp_render_params* p,
     HIPCHK(ctx->nodes.ensure(pl.nodes.size() * sizeof(DevNode)));
     HIPCHK(ctx->defs.ensure(std::max<size_t>(1, sc.ddefs.size()) * sizeof(DevDeform)));
     HIPCHK(ctx->views.ensure(job.views.size() * sizeof(DevView)));
-    // the counters, and the march's tile counter after them
-    HIPCHK(ctx->stats.ensure((ST_COUNT + 1) * sizeof(unsigned long long)));
+    // the counters, the march's tile counter on the next line, and its sink
+    HIPCHK(ctx->stats.ensure(2 * kStatStride * sizeof(unsigned long long) + kBatchSinkBytes));
     HIPCHK(hipMemcpy(ctx->nodes.p, pl.nodes.data(), pl.nodes.size() * sizeof(DevNode),
                      hipMemcpyHostToDevice));
     if (!sc.ddefs.empty())
@@ -2459,11 +2459,11 @@ int xrp_surrogate_render_device(xrp_surrogate* s, const xrp_render_params* p,
     }
     xrp_surrogate_stats out_st;
     std::memset(&out_st, 0, sizeof out_st);
-    HIPCHK(hipMemsetAsync(ctx->stats.p, 0, (ST_COUNT + 1) * sizeof(unsigned long long),
+    HIPCHK(hipMemsetAsync(ctx->stats.p, 0, 2 * kStatStride * sizeof(unsigned long long),
                           ctx->stream));
     MarchParams smp = mp;
     smp.stats = (unsigned long long*)ctx->stats.p;
-    smp.counts = (uint32_t*)(smp.stats + ST_COUNT);
+    smp.counts = (uint32_t*)(smp.stats + kStatStride);
     HIPCHK(hipEventRecord(ctx->ev0, ctx->stream));
     int e = launch_sur_render(s->net, smp, ds_sur, ctx->stream);
     if (e) return fail(XRP_ERR_DEVICE, hipGetErrorString((hipError_t)e));

@@ -267,7 +267,7 @@ struct BatchGroup {
   int32_t line_cap;             // interval march: run slots of the largest job
 };
 // Lines that take the bookkeeping atomics of a wave's lanes other than its
-// first (batch.hip lane_slot).
+// first (eval_device.hpp lane_slot).
 constexpr int kBatchSinkBytes = 64 * 128;
 int launch_batch(const BatchGroup& g, int precision, int integrator, int workgroups,
                  void* stream);

@@ -780,7 +780,8 @@ __device__ __forceinline__ float mlp_density(const SurMlpLds& L, float b3, int l
 
 // RESIDENT: one workgroup a CU, which stays for the launch: it stages the weights and
 // tables once, and its waves take tiles (16 rays, 4x4 pixels) from the counter
-// p.counts until none is left.
+// p.counts until none is left (kStatStride words after it, kBatchSinkBytes that
+// the adds of a wave's other lanes go to).
 //
 // The gathers bound it: 64 lines of a step's 128 corners are distinct for each
 // sample (fine cells are smaller than the pixel spacing), and L1 and L2 are
@@ -839,13 +840,14 @@ __global__ __launch_bounds__(RESIDENT ? 64 * kSurMarchWaves : 64)
   const float dsf = (float)ds_sur;
   unsigned long long n_samples = 0;
 
-  for (bool more = true; more; more = RESIDENT) {
-    unsigned tile = blockIdx.x;
-    if constexpr (RESIDENT) {
-      if (lane == 0) tile = atomicAdd(p.counts, 1u);
-      tile = __builtin_amdgcn_readfirstlane(tile);
-      if (tile >= n_tiles) break;
-    }
+  // the next tile, by an atomic of every lane (eval_device.hpp lane_slot)
+  auto next = [&]() -> unsigned {
+    if constexpr (!RESIDENT) return n_tiles;
+    unsigned long long* sink = (unsigned long long*)p.counts + kStatStride;
+    return __builtin_amdgcn_readfirstlane(
+        atomicAdd(lane_slot(p.counts, sink), first_lane() ? 1u : 0u));
+  };
+  for (unsigned tile = RESIDENT ? next() : blockIdx.x; tile < n_tiles; tile = next()) {
     const int v = (int)(tile / per_view);
     const int in_view = (int)(tile - (unsigned)v * per_view);
     const int ti = in_view / tiles_j, tj = in_view - ti * tiles_j;
