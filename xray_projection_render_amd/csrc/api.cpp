@@ -772,23 +772,30 @@ int copy_to_host(xrp_context* ctx, void* dst, const void* src, size_t bytes) {
 }
 
 // Copies new values into a voxel root's device grid (allocated on first use)
-// and builds the brick copies held for it again.
+// and builds the brick copies held for it again.  The registry is locked for
+// its own entries alone: the caller holds the context, no other uses the scene,
+// and other contexts' renders need the registry while this copy runs (half a
+// gigabyte 14 ms).
 int refresh_volume(xrp_context* ctx, xrp_scene* sc, const float* volume) {
-  std::lock_guard<std::mutex> g(g_registry_mu);
   const xrp::HNode& n = sc->s->root;
   const size_t bytes = (size_t)n.nx * n.ny * n.nz * sizeof(float);
-  auto it = sc->uploads.find(ctx);
-  if (it == sc->uploads.end()) {
-    void* p = nullptr;
-    hipError_t e = hipMalloc(&p, bytes);
-    if (e != hipSuccess)
-      return fail(XRP_ERR_ALLOC, std::string("voxel upload failed: ") + hipGetErrorString(e));
-    std::vector<void*> out(1, p);
-    out.insert(out.end(), N_SLOTS, nullptr);
-    it = sc->uploads.emplace(ctx, std::move(out)).first;
-    ctx->scenes.insert(sc);
+  std::vector<void*> out;
+  {
+    std::lock_guard<std::mutex> g(g_registry_mu);
+    auto it = sc->uploads.find(ctx);
+    if (it == sc->uploads.end()) {
+      void* p = nullptr;
+      hipError_t e = hipMalloc(&p, bytes);
+      if (e != hipSuccess)
+        return fail(XRP_ERR_ALLOC, std::string("voxel upload failed: ") + hipGetErrorString(e));
+      out.assign(1, p);
+      out.insert(out.end(), N_SLOTS, nullptr);
+      sc->uploads.emplace(ctx, out);
+      ctx->scenes.insert(sc);
+    } else {
+      out = it->second;
+    }
   }
-  const std::vector<void*>& out = it->second;
   HIPCHK(hipMemcpyAsync(out[0], volume, bytes, hipMemcpyHostToDevice, ctx->stream));
   for (int slot = 0; slot < N_SLOTS; ++slot)
     if (void* p = out[out.size() - N_SLOTS + slot]) {
