@@ -1102,11 +1102,15 @@ int plan_job(xrp_context* ctx, xrp_scene* sc, const RenderJob& job, LaunchPlan& 
     mp.vbricks[1] = (s.root.ny + 3) / 4;
     mp.vbricks[2] = (s.root.nz + 3) / 4;
     std::vector<void*> q;
+    const std::string said = g_error;
     if ((size_t)mp_bricks(s.root) * 64 < ((size_t)1 << 28) &&
-        upload_voxels(ctx, sc, q, SLOT_QUAD, no_alloc) == XRP_OK)
+        upload_voxels(ctx, sc, q, SLOT_QUAD, no_alloc) == XRP_OK) {
       mp.vgrid = (const float*)q[q.size() - N_SLOTS + SLOT_QUAD];
-    else
+    } else {
+      // no error: the linear copy is read
       (void)hipGetLastError();
+      g_error = said;
+    }
   }
   if (line.line) {
     mp.line = line.line;
