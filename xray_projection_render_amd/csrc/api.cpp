@@ -468,6 +468,13 @@ bool two_pass_forced() {
   return e && std::strcmp(e, "1") == 0;
 }
 
+// Quad copies of voxel roots for FP64 renders (XRP_FP64_QUADS=0 builds none;
+// read per render; the image is the same either way).
+bool fp64_quads_enabled() {
+  const char* e = std::getenv("XRP_FP64_QUADS");
+  return !(e && std::strcmp(e, "0") == 0);
+}
+
 // Per-wave culling of a root collection's children (XRP_CULL=0 turns it
 // off, for comparison; the image is the same either way).
 bool cull_enabled() {
@@ -1089,9 +1096,13 @@ int plan_job(xrp_context* ctx, xrp_scene* sc, const RenderJob& job, LaunchPlan& 
     // FP32 anchor rounding (u*|G|) plus the FP32 step (4u * |B| * chunk*ds).
     mp.vguard = (float)(4.0 * (u * (N + 4.0 * L * 0.5 * N * 32.0 * job.ds) + 1e-9));
   }
-  // FP64 marches of a voxel root read its quad bricks (built on first use;
-  // for a launch without allocation, where they are there already), or the
-  // linear copy where the quads would pass 4 GiB or have no room
+  // FP64 marches of a voxel root read its quad bricks where they are there
+  // already, and otherwise build them, four times the grid that then stays with
+  // the scene, or read the linear copy (12 x 256^2 of 120 x 100 x 90 voxels 0.51
+  // ms against 0.33).  The copy is built for renders that come again: not under
+  // audit, not for a launch without allocation, not past 4 GiB nor an eighth of
+  // the memory that is free (the program's next allocations have no fallback),
+  // and not with $XRP_FP64_QUADS=0.
   if (allow_voxel_kernel && s.root.kind == K_VOXEL && !vox_kernel &&
       precision == XRP_PRECISION_FP64) {
     mp.vlin = (const float*)vptr.front();
@@ -1103,8 +1114,17 @@ int plan_job(xrp_context* ctx, xrp_scene* sc, const RenderJob& job, LaunchPlan& 
     mp.vbricks[2] = (s.root.nz + 3) / 4;
     std::vector<void*> q;
     const std::string said = g_error;
+    auto quads = [&](bool resident) {
+      return upload_voxels(ctx, sc, q, SLOT_QUAD, resident) == XRP_OK;
+    };
+    auto room = [&] {
+      size_t free = 0, total = 0;
+      return hipMemGetInfo(&free, &total) == hipSuccess &&
+             brick_bytes(s.root, SLOT_QUAD) <= free / 8;
+    };
     if ((size_t)mp_bricks(s.root) * 64 < ((size_t)1 << 28) &&
-        upload_voxels(ctx, sc, q, SLOT_QUAD, no_alloc) == XRP_OK) {
+        (quads(true) ||
+         (!no_alloc && !job.audit && fp64_quads_enabled() && room() && quads(false)))) {
       mp.vgrid = (const float*)q[q.size() - N_SLOTS + SLOT_QUAD];
     } else {
       // no error: the linear copy is read
