@@ -1275,6 +1275,8 @@ int render_core(xrp_context* ctx, xrp_scene* sc, const RenderJob& job,
   // the lists, sized for the largest launch (XRP_DEFER_CAP and
   // XRP_REDO_CAP shorten them, for tests: 1 and up)
   TwoPassCaps caps = two_pass_caps(two_pass ? (size_t)std::min(vpc, nv) * res * res : 0, hier);
+  // the interval march's first pass lists rays to march again and nothing else
+  if (line) caps.defer = caps.k = 0;
   if (const char* e = std::getenv("XRP_DEFER_CAP"))
     caps.defer = (uint32_t)std::min<long>(caps.defer, std::max(1L, std::atol(e)));
   if (const char* e = std::getenv("XRP_REDO_CAP"))
