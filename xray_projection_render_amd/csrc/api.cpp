@@ -515,6 +515,90 @@ bool compose_linear(const std::vector<xrp::HDeform>& defs, double M[9], double t
   return true;
 }
 
+// Whether a convex primitive holds a point.
+bool convex_holds(const xrp::HNode& n, const double x[3]) {
+  double w[3];
+  for (int k = 0; k < 3; ++k) w[k] = x[k] - n.c[k];
+  switch (n.kind) {
+    case xrp::K_SPHERE: return w[0] * w[0] + w[1] * w[1] + w[2] * w[2] <= n.a * n.a;
+    case xrp::K_BOX:
+      return std::fabs(w[0]) <= 0.5 * n.v[0] && std::fabs(w[1]) <= 0.5 * n.v[1] &&
+             std::fabs(w[2]) <= 0.5 * n.v[2];
+    case xrp::K_PPED:
+      for (int i = 0; i < 3; ++i) {
+        const double t = n.minv[i] * w[0] + n.minv[3 + i] * w[1] + n.minv[6 + i] * w[2];
+        if (!(t >= 0.0 && t <= 1.0)) return false;
+      }
+      return true;
+    case xrp::K_CYL: {
+      double t = 0, vv = 0, ww = 0;
+      for (int k = 0; k < 3; ++k) {
+        const double v = n.v[k] - n.c[k];
+        t += w[k] * v, vv += v * v, ww += w[k] * w[k];
+      }
+      return t >= 0.0 && t <= vv && ww - t * t / vv <= n.a * n.a;
+    }
+  }
+  return false;
+}
+
+// A point inside a convex primitive: its centre, of a cylinder the one on its
+// axis nearest to x.
+void convex_centre(const xrp::HNode& n, const double x[3], double c[3]) {
+  for (int k = 0; k < 3; ++k) c[k] = n.c[k];
+  if (n.kind == xrp::K_PPED) {
+    for (int k = 0; k < 3; ++k) c[k] += 0.5 * (n.pv[k] + n.pv[3 + k] + n.pv[6 + k]);
+  } else if (n.kind == xrp::K_CYL) {
+    double t = 0, vv = 0;
+    for (int k = 0; k < 3; ++k) {
+      t += (x[k] - n.c[k]) * (n.v[k] - n.c[k]);
+      vv += (n.v[k] - n.c[k]) * (n.v[k] - n.c[k]);
+    }
+    t = std::min(std::max(t / vv, 0.0), 1.0);
+    for (int k = 0; k < 3; ++k) c[k] += t * (n.v[k] - n.c[k]);
+  }
+}
+
+// About how many convex children of a collection one place of a wave's pencil
+// of rays meets: of 8 places (centres of children), the most children, of at
+// most 64 and scaled up, that hold a point within h of it across the ray's
+// direction there.
+double pencil_depth(const xrp::HNode* kids, size_t n, const RenderJob& job, const double M[9],
+                    double h) {
+  const int places = 8;
+  const size_t stride = (n + 63) / 64;
+  double most = 0;
+  for (int q = 0; q < places; ++q) {
+    const xrp::DevView& v = job.views[(size_t)q * job.views.size() / places];
+    const xrp::HNode& at = kids[(2 * (size_t)q + 1) * n / (2 * places)];
+    if (at.kind == xrp::K_GYROID) continue;
+    double d[3], u[3], len = 0, x[3];
+    for (int k = 0; k < 3; ++k) d[k] = -v.cam[4 * k + 2];
+    for (int k = 0; k < 3; ++k) {
+      u[k] = M[3 * k] * d[0] + M[3 * k + 1] * d[1] + M[3 * k + 2] * d[2];
+      len += u[k] * u[k];
+    }
+    for (int k = 0; k < 3; ++k) u[k] /= std::sqrt(len);
+    convex_centre(at, at.c, x);
+    size_t held = 0, tried = 0;
+    for (size_t i = (size_t)q % stride; i < n; i += stride, ++tried) {
+      if (kids[i].kind == xrp::K_GYROID) continue;
+      double c[3], a = 0, l = 0;
+      convex_centre(kids[i], x, c);
+      for (int k = 0; k < 3; ++k) a += (c[k] -= x[k]) * u[k];
+      for (int k = 0; k < 3; ++k) {
+        c[k] -= a * u[k];
+        l += c[k] * c[k];
+      }
+      const double go = l > h * h ? h / std::sqrt(l) : 1.0;
+      for (int k = 0; k < 3; ++k) c[k] = x[k] + go * c[k];
+      held += convex_holds(kids[i], c) ? 1 : 0;
+    }
+    if (tried) most = std::max(most, (double)held * (double)n / (double)tried);
+  }
+  return most;
+}
+
 // Whether the interval march (line_march.hpp) takes a scene, and with what:
 // the object-space map must be affine and well conditioned, and the tree one
 // primitive, a collection of them, or a tessellation of a collection of
@@ -563,7 +647,7 @@ bool line_plan(const xrp::Scene& s, const RenderJob& job, double lip, double s_e
     n_kids = c.kids.size();
   }
   if (n_kids == 0 || s.nodes.size() > 32767) return false;
-  double cell = 0.0;
+  double cell = 0.0, narrowest = INFINITY;
   if (tess) {
     for (int k = 0; k < 3; ++k) {
       const double d = root.ucb[2 * k + 1] - root.ucb[2 * k];
@@ -614,6 +698,7 @@ bool line_plan(const xrp::Scene& s, const RenderJob& job, double lip, double s_e
         // path length 2 * half diagonal over the period 2 pi scale
         if (!(6.2831853 * n.a >= lip * kCubeHalfDiagonal)) return false;
         ++gyroids;
+        narrowest = std::min(narrowest, n.a);
         least = INFINITY;
         break;
       default: return false;
@@ -622,6 +707,13 @@ bool line_plan(const xrp::Scene& s, const RenderJob& job, double lip, double s_e
       if (!std::isfinite(n.c[k])) return false;
     if (!(least >= 1e-9 * W) || !std::isfinite(n.rho)) return false;
   }
+  // Many narrow gyroids at coarse steps: each costs about as many evaluations as
+  // its level has crossings, however few samples the sampling march makes.  48
+  // and 60 gyroids of thickness 0.3, 4 x 256^2 rays, period 1.76: step 0.004 8.5
+  // and 13.0 against 34 and 47 ms, 0.03 (59 samples a period) 5.8 and 8.8 against
+  // 6.2 and 7.8, 0.08 4.1 and 6.4 against 2.7 and 3.1; period 3.1 at 0.03 3.4 and
+  // 5.0 against 6.2 and 7.8.  20 gyroids gain at all of them.
+  if (gyroids > 24 && !(6.2831853 * narrowest >= 64.0 * lip * job.ds)) return false;
   std::memcpy(mp.M, M, sizeof M);
   std::memcpy(mp.t, t, sizeof t);
   mp.line = tess ? LINE_TESS : LINE_COLL;
@@ -632,11 +724,41 @@ bool line_plan(const xrp::Scene& s, const RenderJob& job, double lip, double s_e
   // per CU) take a slot per possible run: their wide pencils of rays meet
   // most children, and nothing competes for the LDS.
   const size_t need = n_kids + 2 * gyroids;
-  const size_t tiles = (size_t)((job.res + 7) / 8) * (size_t)((job.res + 7) / 8) * job.views.size();
-  const size_t cap = tiles <= 1024 && !job.batched ? (size_t)kLineCapMost
-                     : n_kids <= 64 ? (size_t)kLineCap
-                     : n_kids <= 128 ? 2 * (size_t)kLineCap : 3 * (size_t)kLineCap;
-  mp.line_cap = tess ? (int)n_kids : (int)std::min(cap, need);
+  if (tess) {
+    mp.line_cap = (int)n_kids;
+  } else {
+    const size_t tiles =
+        (size_t)((job.res + 7) / 8) * (size_t)((job.res + 7) / 8) * job.views.size();
+    size_t cap = tiles <= 1024 && !job.batched ? (size_t)kLineCapMost
+                 : n_kids <= 64 ? (size_t)kLineCap
+                 : n_kids <= 128 ? 2 * (size_t)kLineCap : 3 * (size_t)kLineCap;
+    // A place that more children hold than there are slots is halved down to
+    // single indices, each of which computes every child's runs: 4 x 256^2 rays
+    // through 60 overlapping spheres, step 0.004, 32 slots 17.3 ms, 60 slots
+    // 0.49, sampling march 3.9; hierarchical at 0.02 36, 0.60 and 1.27; 180
+    // spheres, 96 slots 47.5, 180 slots 2.7, sampling 11.7.  So the slots follow
+    // the children that overlap, twice their number and 8 (60 spheres of radius
+    // 0.15 to 0.3, 8 x 128^2: 32 slots 2.6 ms, an eighth more than overlap and 8
+    // 0.48, twice 0.29, sampling 3.5); a gyroid, unbounded and with several runs,
+    // counts for one and a half (60 of half a period, 32 slots 27.7 ms, 64 13.0,
+    // 128 18.7, sampling 46).  Where not even an eighth more than overlap fit, past
+    // 128 of them with the hierarchical integrator (180 spheres 3.9 ms, sampling
+    // 3.7), and in a batch past 96 slots, the sampling march is taken.
+    if (need > 48) {
+      const double f = 1.0 / std::tan(job.fov * M_PI / 360.0);
+      const double h = 4.0 * M_SQRT2 * lip * 2.0 * std::fabs(job.R) / (f * job.res);
+      const double over = pencil_depth(kids, n_kids, job, M, h), runs = 1.5 * (double)gyroids;
+      const double least = std::min((double)need, 1.125 * (over + runs) + 8.0);
+      const double limit = job.batched ? 3.0 * kLineCap : (double)kLineCapMost;
+      if (least > limit || (job.integrator == XRP_INTEGRATE_HIERARCHICAL && least > 152.0))
+        return false;
+      const double slots = std::max(least, 2.0 * over + 1.125 * runs + 8.0);
+      cap = std::max(cap, (size_t)std::min(slots, limit));
+    } else {
+      cap = std::max(cap, need);
+    }
+    mp.line_cap = (int)std::min(cap, need);
+  }
   mp.line_cap = (mp.line_cap + 3) & ~3;  // whole groups (line_scan)
   // FP64 roundings of positions through the chain (64 ulps of the reach), the
   // sample table's drift, and, for cells, FP32 cell-local coordinates
