@@ -8,16 +8,14 @@
 
 namespace xrp {
 
+// Adds the wave's sum of v; nothing, on a wave-uniform condition, where it is
+// zero.
 __device__ __forceinline__ void wave_add(unsigned long long* p, unsigned long long v,
                                          unsigned long long* sink) {
+  if (!__ballot(v != 0ull)) return;
+  v = wave_sum(v);
   atomicAdd(lane_slot(p, sink), first_lane() ? v : 0ull);
 }
-
-// Items a wave takes per counter operation.  A wave adds its stats and its
-// scene's last-end stamp once per run of consecutive items of one scene
-// (items are queued scene by scene), so a one-scene batch costs a quarter
-// of the same-address operations per item.
-constexpr uint32_t kItemsPerGrab = 4;
 
 // Close a wave's run of items of scene `job`: its stats, once, and its
 // last-end stamp.  All conditions are wave-uniform (job and p.stats are).
@@ -26,11 +24,11 @@ __device__ __forceinline__ void close_run(const BatchGroup& g,
                                           const RayCounts& rc) {
   const MarchParams& p = jobs[job];
   if (p.stats) {
-    wave_add(p.stats + ST_SAMPLES, wave_sum(rc.samples), g.sink);
-    wave_add(p.stats + ST_REEVAL, wave_sum(rc.reeval), g.sink);
-    wave_add(p.stats + ST_AUDIT_MISS, wave_sum(rc.miss), g.sink);
-    wave_add(p.stats + ST_FINE, wave_sum(rc.fine), g.sink);
-    wave_add(p.stats + ST_SKIPPED, wave_sum(rc.skipped), g.sink);
+    wave_add(p.stats + ST_SAMPLES, rc.samples, g.sink);
+    wave_add(p.stats + ST_REEVAL, rc.reeval, g.sink);
+    wave_add(p.stats + ST_AUDIT_MISS, rc.miss, g.sink);
+    wave_add(p.stats + ST_FINE, rc.fine, g.sink);
+    wave_add(p.stats + ST_SKIPPED, rc.skipped, g.sink);
   }
   atomicMax(lane_slot(g.t_done + job, g.sink), (unsigned long long)wall_clock64());
 }

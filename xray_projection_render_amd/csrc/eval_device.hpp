@@ -787,17 +787,22 @@ __device__ __forceinline__ unsigned long long wave_total(unsigned long long v) {
 // inside the persistent loop (no lane-conditional blocks next to the loop's
 // back edge, where a divergent branch could split one wave's lanes across
 // loop iterations; a lane-0-only form faulted for that reason).  Only the
-// first active lane targets the real address; every other lane hits a line
-// of its own in the sink, so an item costs one same-address operation per
-// counter instead of 64 (a one-scene batch of 8192 items: 3.2 us per item,
-// serialized on its scene's counters).
+// first active lane targets the real address; the others add to a word each of
+// the sink, so an item costs one same-address operation per counter instead of
+// 64 (a one-scene batch of 8192 items: 3.2 us per item, serialized on its
+// scene's counters).  The words of a wave are neighbours, one request per line
+// of 16, and 16 blocks of workgroups have a part of the sink each.  With a line
+// per lane an atomic was 64 requests, and 1.2 million of them bounded batches
+// of simple scenes: one sphere, 8 x 256^2, 8192 items, hierarchical, interval
+// march 407 us, sampling march 235; now 263 and 171, and with no adds of zero
+// (batch_items.hpp wave_add) 72 and 75.
 __device__ __forceinline__ bool first_lane() {
   return __builtin_amdgcn_readfirstlane((int)(threadIdx.x & 63)) == (int)(threadIdx.x & 63);
 }
 
 template <typename T>
 __device__ __forceinline__ T* lane_slot(T* real, unsigned long long* sink) {
-  return first_lane() ? real : (T*)(sink + 16 * (threadIdx.x & 63));
+  return first_lane() ? real : (T*)(sink + 64 * (blockIdx.x & 15) + (threadIdx.x & 63));
 }
 
 }  // namespace xrp

@@ -260,15 +260,20 @@ struct BatchGroup {
   uint32_t* counter;            // work counter, zeroed by launch_batch_reset
   unsigned long long* t_first;  // per job: wall clock at its first tile start
   unsigned long long* t_done;   // per job: wall clock at its last tile end
-  unsigned long long* sink;     // kBatchSinkBytes: one 128-byte line per lane
+  unsigned long long* sink;     // kBatchSinkBytes
   int32_t n_jobs;
   uint32_t n_tiles;
   int32_t wave_rows, wave_cols; // item: (8 wave_rows) x (8 wave_cols) pixels, one wave
   int32_t line_cap;             // interval march: run slots of the largest job
 };
-// Lines that take the bookkeeping atomics of a wave's lanes other than its
+// Items a wave takes per counter operation.  A wave adds its stats and its
+// scene's last-end stamp once per run of consecutive items of one scene
+// (items are queued scene by scene), so a one-scene batch costs a quarter
+// of the same-address operations per item.
+constexpr uint32_t kItemsPerGrab = 4;
+// Words that take the bookkeeping atomics of a wave's lanes other than its
 // first (eval_device.hpp lane_slot).
-constexpr int kBatchSinkBytes = 64 * 128;
+constexpr int kBatchSinkBytes = 16 * 64 * 8;
 int launch_batch(const BatchGroup& g, int precision, int integrator, int workgroups,
                  void* stream);
 // The same for a group whose jobs take the interval march (line != LINE_NONE);
