@@ -972,7 +972,7 @@ int refresh_volume(xrp_context* ctx, xrp_scene* sc, const float* volume) {
 // 512^2 36 us), and the tests of the deferral lists (tests/test_gpu_two_pass.py)
 // need rays with several of them: at 1.05, 32 rays of 8192 had one and none two.
 int gyroid_plan(const xrp::Scene& s, const std::vector<xrp::DevNode>& nodes, double delta,
-                bool simple, xrp::MarchParams& mp) {
+                bool simple, double ds, xrp::MarchParams& mp) {
   using namespace xrp;
   const char* e = std::getenv("XRP_GYROID");
   if (e && std::strcmp(e, "0") == 0) return 0;
@@ -982,6 +982,19 @@ int gyroid_plan(const xrp::Scene& s, const std::vector<xrp::DevNode>& nodes, dou
   const DevNode &t = nodes[0], &g = nodes[2];
   if (!(g.d[3] > 0.0) || !std::isfinite(g.d[4])) return 0;
   const double period = 2.0 * M_PI * g.d[3];
+  const bool tanh = s.ddefs.size() == 1 && s.ddefs[0].kind == D_TANH;
+  // Hierarchical, with coarse steps about as long as a cell: every step has a
+  // density change, so there is nothing to settle, and the lanes of a wave wait
+  // for each other at guard-band samples, in the slow FP64 form of a general
+  // chain.  Sigmoid displacement, 2 x 24^2 rays, thickness 0.5, general march
+  // against this: 0.6 steps a cell 0.104 against 0.138 ms, 1.25 0.103 and 0.144,
+  // 6.3 0.45 and 0.51, 12.5 0.36 and 0.29; without a chain 0.6 0.089 and 0.096,
+  // 1.25 0.090 and 0.091, 6.3 0.36 and 0.25.
+  if (!simple) {
+    const double steps = s.ddefs.empty() || tanh ? 1.0 : 8.0;
+    for (int a = 0; a < 3; ++a)
+      if (!(t.d[9 + a] - t.d[6 + a] >= steps * ds)) return 0;
+  }
   double bb = 0.0;
   for (int k = 0; k < 6; ++k) bb = std::max(bb, std::fabs(t.d[k]));
   for (int a = 0; a < 3; ++a) {
@@ -996,7 +1009,7 @@ int gyroid_plan(const xrp::Scene& s, const std::vector<xrp::DevNode>& nodes, dou
   const double eq = (delta + u * (2.0 * bb + 2.0 * cm)) / g.d[3] + 2.0 * M_PI * u;
   const double kappa = simple ? 4.0 : 1.05;
   mp.gyro_band = (float)(kappa * (3.07 * eq + 6.0 * kHwSinCosErr + 16.0 * u));
-  mp.gyro_tanh = s.ddefs.size() == 1 && s.ddefs[0].kind == D_TANH ? 1 : 0;
+  mp.gyro_tanh = tanh ? 1 : 0;
   const double rho = g.d[5];
   mp.gyro_rho = nodes[1].greedy && rho > 0.0 ? rho : rho < 0.0 ? 0.0 : rho > 1.0 ? 1.0 : rho;
   const double rr = mp.gyro_rho * mp.dm;
@@ -1133,7 +1146,8 @@ int plan_job(xrp_context* ctx, xrp_scene* sc, const RenderJob& job, LaunchPlan& 
       for (const auto& n : pl.nodes)
         if (n.kind == K_GYROID && n.g[6] > 0.0f) mp.vel = 1;
   }
-  mp.gyro = gyroid_plan(s, pl.nodes, delta, job.integrator == XRP_INTEGRATE_SIMPLE, mp);
+  mp.gyro =
+      gyroid_plan(s, pl.nodes, delta, job.integrator == XRP_INTEGRATE_SIMPLE, job.ds, mp);
   // Samples per node visit of the per-scene guarded simple march: with the
   // safe radius, 2 is faster on small trees (lattice cell 10 nodes: 6 %
   // faster than 1), 4 on large collections, whose node walk it amortises
