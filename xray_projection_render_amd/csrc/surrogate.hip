@@ -17,6 +17,7 @@
 
 #include <algorithm>
 #include <cmath>
+#include <cstdlib>
 #include <type_traits>
 
 #include "eval_device.hpp"
@@ -1002,17 +1003,24 @@ int launch_sur_labels(const SurNet& net, const MarchParams& scene, uint64_t seed
 
 static int64_t sur_train_chunk(int64_t n) { return std::min(n, kSurTrainChunk); }
 
+// Whether the tables' gradients are added by slices ($XRP_SUR_SLICES: fewer
+// slices at most, for tests; read per batch).
+static bool sur_sliced(const SurNet& net) {
+  uint32_t most = kSurSlicesMost;
+  if (const char* e = std::getenv("XRP_SUR_SLICES"))
+    most = (uint32_t)std::min<long>(most, std::max(0L, std::atol(e)));
+  return sur_slices(net) <= most;
+}
+
 size_t sur_train_bytes(const SurNet& net, int64_t n) {
   const size_t sums = (size_t)kSurTrainGroups * kSurMlpParams * sizeof(float);
-  return sums + (sur_slices(net) <= kSurSlicesMost
-                     ? (size_t)sur_train_chunk(n) * kSurLevels * sizeof(float2)
-                     : 0);
+  return sums + (sur_sliced(net) ? (size_t)sur_train_chunk(n) * kSurLevels * sizeof(float2) : 0);
 }
 
 int launch_sur_train(const SurNet& net, const float* pts, const float* labels, int64_t n,
                      float inv_n, float* grads, double* loss_sum, void* work, void* stream) {
   const uint32_t slices = sur_slices(net);
-  float2* dx = slices <= kSurSlicesMost ? (float2*)work : nullptr;
+  float2* dx = sur_sliced(net) ? (float2*)work : nullptr;
   float* sums = (float*)work + (dx ? (size_t)sur_train_chunk(n) * kSurLevels * 2 : 0);
   hipStream_t s = (hipStream_t)stream;
   for (int64_t at = 0; at < n; at += kSurTrainChunk) {
