@@ -147,3 +147,17 @@ def test_batch_of_overlaps(ctx, monkeypatch):
         ref = oracle_render(oracle_scene(objs[k]), ANGLES, 24, 0.02, integrator="simple")
         assert float(np.abs(got[k].astype(np.float64) - ref).max()) <= 1e-5, k
         sc.close()
+
+
+def test_batch_keeps_scenes_of_many_gyroids(ctx):
+    """A place has at most one run of each gyroid, so 60 of them fit the 96 slots
+    of a batch, where the sampling march of one such scene outlasts all others."""
+    objs = [_overlapping(60), _gyroids(60, 1.0)]
+    scenes = [xrp_scene(o) for o in objs]
+    b = X.Batch(ctx, [(sc, ANGLES, 24, 0.02, {"integrator": "simple"}) for sc in scenes])
+    assert b.run()["launches"] == 1
+    for k, sc in enumerate(scenes):
+        ref = oracle_render(oracle_scene(objs[k]), ANGLES, 24, 0.02, integrator="simple")
+        assert float(np.abs(b.read(k).astype(np.float64) - ref).max()) <= 1e-5, k
+        sc.close()
+    b.close()
