@@ -463,9 +463,10 @@ bool reach_enabled() {
   return on;
 }
 
-// Two-pass guarded simple march (XRP_TWO_PASS=0 turns it off, for
-// comparison; 1 takes it for small jobs too, for tests; read per render;
-// the image is the same either way).
+// Two-pass guarded marches (XRP_TWO_PASS=0 turns them off, for comparison; 1
+// takes them for small jobs too, for tests; read per render; the sampling and
+// gyroid marches' images are the same either way.  Any setting also leaves the
+// interval march's scenes to the sampling marches: line_plan).
 bool two_pass_enabled() {
   const char* e = std::getenv("XRP_TWO_PASS");
   return !(e && std::strcmp(e, "0") == 0);
@@ -1357,6 +1358,15 @@ int render_core(xrp_context* ctx, xrp_scene* sc, const RenderJob& job,
   // launches cost more than they save: CSG 8 x 256^2 0.107 against 0.097
   // ms).  A launch covers at most 2^31 rays, which the lists name by 32-bit
   // index.  Not under audit, nor without allocation.
+  // The interval march (simple) lists the rays a tie stops.  They are few, and
+  // the second pass costs its launch and the time of one such ray: strut lattice
+  // 4 x 512^2, 4 and 16 x 1024^2 one pass 0.237, 0.418 and 1.43 ms, two 0.246,
+  // 0.445 and 1.47; 60 spheres 4 x 1024^2 0.157 against 0.153, with one ray
+  // listed 0.159 against 0.227.  Views along cell faces stop whole columns, which
+  // one pass takes up ray by ray in the wave that met them: 0.76 and 1.73 ms at 4
+  // and 16 x 1024^2, two 0.21 and 0.66.  So large jobs, where that wave would
+  // outlast the others, take two, and small ones one, though along faces they
+  // too would gain (4 x 256^2 0.79 against 0.10).
   const int kMaxGridY = 65535;
   const bool hier = job.integrator == XRP_INTEGRATE_HIERARCHICAL;
   const bool line = pl.mp.line != LINE_NONE;
@@ -2313,7 +2323,7 @@ struct xrp_surrogate {
   int64_t table_count = 0;  // of which tables
   DevBuf params, grads, m, v, tbf16, loss, pts, labels, scene_nodes, items, vals;
   DevBuf judge, counters;  // certified check: exact images, tile counters
-  DevBuf work;             // training: at most 33 MiB (sur_train_bytes)
+  DevBuf work;             // training: at most 23 MiB (sur_train_bytes)
   int adam_step = 0;
   bool packed = false;
   ~xrp_surrogate() {

@@ -34,8 +34,9 @@ __device__ __forceinline__ void close_run(const BatchGroup& g,
 }
 
 // Every wave of a persistent grid takes items until the counter passes the
-// last one (no LDS, no barriers); march(p, v, i, j, valid, rc) renders one
-// pixel per lane, called by every lane of the wave.
+// last one, without LDS or barriers of the loop's own (the interval march keeps
+// a wave's run slots and child list in LDS, line.hip); march(p, v, i, j, valid,
+// rc) renders one pixel per lane, called by every lane of the wave.
 template <class March>
 __device__ __forceinline__ void batch_items(const BatchGroup& g,
                                             const MarchParams* __restrict__ jobs, March&& march) {
