@@ -1295,10 +1295,11 @@ int plan_job(xrp_context* ctx, xrp_scene* sc, const RenderJob& job, LaunchPlan& 
     auto quads = [&](bool resident) {
       return upload_voxels(ctx, sc, q, SLOT_QUAD, resident) == XRP_OK;
     };
-    auto room = [&] {
+    auto room = [&] {  // asking costs up to 60 us: not for small copies
+      const size_t bytes = brick_bytes(s.root, SLOT_QUAD);
       size_t free = 0, total = 0;
-      return hipMemGetInfo(&free, &total) == hipSuccess &&
-             brick_bytes(s.root, SLOT_QUAD) <= free / 8;
+      return bytes <= ((size_t)64 << 20) ||
+             (hipMemGetInfo(&free, &total) == hipSuccess && bytes <= free / 8);
     };
     if ((size_t)mp_bricks(s.root) * 64 < ((size_t)1 << 28) &&
         (quads(true) ||
