@@ -269,6 +269,12 @@ def bench_batch(args) -> int:
     value = pixels / (512.0 * 512.0) / (ms_per_step / 1000.0)
     k_ms = float(np.mean(kms))
     achieved = flops / (k_ms / 1000.0) / 1e12
+    # every scene of the batch takes the interval march, in one launch, unless it is
+    # turned off or leaves some to the sampling march's group
+    kernels = (["batch_kernel<PREC_GUARDED,INT_SIMPLE>"]
+               if os.environ.get("XRP_INTERVALS") == "0" else
+               ["batch_line_kernel<0>", "batch_kernel<PREC_GUARDED,INT_SIMPLE>"])
+    kernel = " + ".join(kernels[:st["launches"]])
     ds_rule = ("MinFeatureSize/5" if args.batch_ds == "reference"
                else f"max(MinFeatureSize/5, {BATCH_MIN_DS})")
     line = {
@@ -287,16 +293,15 @@ def bench_batch(args) -> int:
                        "p99": float(np.percentile(lat, 99)), "max": float(lat.max())},
         "roofline": {"bound": "valu", "achieved": achieved, "peak": FP32_PEAK_TFLOPS,
                      "unit": "TFLOP/s", "frac": achieved / FP32_PEAK_TFLOPS,
-                     "traffic": measured_traffic("batch_kernel<PREC_GUARDED,INT_SIMPLE>",
-                                                 "batch"),
-                     "kernel": "batch_kernel<PREC_GUARDED,INT_SIMPLE>", "kernel_ms": k_ms,
+                     "traffic": measured_traffic(kernel, "batch"),
+                     "kernel": kernel, "kernel_ms": k_ms,
                      "per_sample": "cost table per scene", "samples_per_launch": samples},
     }
     if args.batch_ds == "floored":
         valu_issue(line["roofline"], "batch")
     if line["roofline"]["frac"] > 1.0:
-        line["roofline"]["note"] = ("the cost-table rate counts the samples a safe radius "
-                                    "settles without evaluating them, so it can pass the peak")
+        line["roofline"]["note"] = ("the cost-table rate counts samples that are settled without "
+                                    "evaluating them, so it can pass the peak")
     if not args.no_cpu:
         line["cpu_baseline"] = batch_cpu_baseline(ws)
     print(json.dumps(line))
@@ -414,9 +419,9 @@ def bench_surrogate(args) -> int:
                            "fraction_above_tolerance": frac_over, "tolerance": tol},
         "roofline": {"bound": "mfma", "achieved": achieved, "peak": BF16_PEAK_TFLOPS,
                      "unit": "TFLOP/s", "frac": achieved / BF16_PEAK_TFLOPS,
-                     "traffic": measured_traffic("sur_render_kernel",
+                     "traffic": measured_traffic("sur_render_kernel<true>",
                                                  f"surrogate {n_views} views"),
-                     "kernel": "sur_render_kernel", "kernel_ms": pure["surrogate_ms"],
+                     "kernel": "sur_render_kernel<true>", "kernel_ms": pure["surrogate_ms"],
                      "per_sample": f"{SURROGATE_FLOPS_PER_SAMPLE:.0f} flop (MLP)",
                      "samples_per_launch": sur_samples},
     }
@@ -427,14 +432,22 @@ def bench_surrogate(args) -> int:
     return 0
 
 
+# Wave instructions a second that the 1024 SIMDs issue at 2 cycles each, which FP32
+# multiply-adds, integer adds and moves take at 2.4 GHz (measured 1.01e12 to 1.18e12;
+# minimum, compare, select, shift, conversion and FP64 take 4 cycles, transcendentals
+# 8: profiles/valu_issue_rates.md).
+VALU_PEAK_WAVE_INSTS = 1024 * 2.4e9 / 2
+
+
 def valu_issue(roof: dict, workload: str) -> None:
-    """Executed VALU issue of the roofline's kernel, from the VALU
-    instructions per launch a rocprofv3 summary under profiles/ records
-    (wave instructions x 4 cycles over the 1024 SIMDs' cycles at 2.4 GHz in
-    the measured launch time), when one does."""
+    """VALU instructions a second of the roofline's kernel, from the instructions
+    per launch a rocprofv3 summary under profiles/ records, when one does, and
+    their share of the fastest issue rate.  A kernel reaches 1 with 2-cycle
+    instructions alone."""
     insts = measured_counter("valu_insts_per_launch", roof["kernel"], workload)
     if insts and roof.get("kernel_ms"):
-        roof["valu_issue_frac"] = insts * 4.0 / (roof["kernel_ms"] / 1000.0 * 1024 * 2.4e9)
+        roof["valu_insts_per_s"] = insts / (roof["kernel_ms"] / 1000.0)
+        roof["valu_issue_frac"] = roof["valu_insts_per_s"] / VALU_PEAK_WAVE_INSTS
 
 
 def measured_counter(name: str, kernel: str, workload: str):
@@ -637,7 +650,7 @@ def c5_surrogate_leg(args, ctx, sc, w, exact, kw, plain_ms: float) -> dict:
             gb = st["network_samples"] * SURROGATE_GATHER_BYTES / net_s / 1e9
             out[mode]["roofline"] = {
                 "bound": "mfma", "achieved": tf, "peak": BF16_PEAK_TFLOPS, "unit": "TFLOP/s",
-                "frac": tf / BF16_PEAK_TFLOPS, "kernel": "sur_render_kernel",
+                "frac": tf / BF16_PEAK_TFLOPS, "kernel": "sur_render_kernel<true>",
                 "kernel_ms": st["surrogate_ms"],
                 "gathers": {"achieved": gb, "unit": "GB/s", "l2_peak_measured": l2,
                             "frac": gb / l2 if l2 > 0 else None}}
