@@ -4,8 +4,10 @@
 // chain.  The scene is then one periodic level set inside a box, and a march
 // over it needs none of the node walk of eval_block.hpp.
 //
-// The march is bound by VALU issue (hierarchical first pass: 100 % of the
-// issue slots), so everything per visit
+// The march is bound by VALU issue (first passes: 7.1e11 instructions a second,
+// 57 % of the rate of 2-cycle instructions, with a visit's 12 transcendentals of 8
+// cycles, selects and minima of 4 between; waves wait for issue half their
+// cycles and more, for anything else 7 to 15 %), so everything per visit
 // that does not depend on the sample is hoisted, the cell wrap is left out
 // (the phase is reduced to [-0.5, 0.5] periods anyway, exactly, by one fma
 // against the rounded period count), and each lane runs its own state
@@ -23,7 +25,7 @@
 // about one to evaluate where the walk took four or five visits.
 //
 // Sheared 6^3 gyroid cells against the general march: 16 x 512^2 rays at step
-// 0.001, simple, 1.60 -> 0.54 ms; 24 x 1024^2, hierarchical, 17.0 -> 3.75 ms
+// 0.001, simple, 1.58 -> 0.53 ms; 24 x 1024^2, hierarchical, 17.1 -> 3.84 ms
 // (first pass 12.8 -> 3.15, the FP64 passes 4.0 -> 0.54).
 //
 // Sums: every term is (rho * dm) * ds of one density value, so T is a number

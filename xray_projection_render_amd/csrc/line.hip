@@ -2,15 +2,16 @@
 // of convex primitives (and wide gyroids) seen along straight object-space
 // lines.
 //
-// Bound by VALU issue and, on collections, by the latency of its serial
-// chains (VALU issue 38 % at 3-4 waves per SIMD): the runs of every listed
-// child (about 80 FP32 instructions each) and one pass over the wave's run
-// slots per change of the density, where the sampling marches evaluated
-// every listed child at every sample they could not settle.  Whole calls,
-// sampling march -> interval march: strut lattice 30 x 500^2 6.81 -> 1.02
-// ms, hierarchical bytes 12 x 512^2 10.2 -> 1.16 ms; 60 primitives
-// hierarchical 8 x 256^2 6.34 -> 0.52 ms; three primitives 2 x 128^2 0.100
-// -> 0.043 ms; 10 uneven scenes batched 21.5 -> 2.75 ms.
+// Bound by VALU issue on tessellations (6.1e11 instructions a second, half the
+// rate of 2-cycle instructions with the roots' minima, selects and
+// transcendentals between) and, on collections, by the latency of serial chains
+// (2.2e11, 3 waves per SIMD): the runs of every listed child (about 80 FP32
+// instructions each) and one pass over the wave's run slots per change of the
+// density, where the sampling marches evaluated every listed child at every
+// sample they could not settle.  Whole calls, sampling march -> interval march:
+// strut lattice 30 x 500^2 7.39 -> 0.88 ms, hierarchical bytes 12 x 512^2 10.0 ->
+// 1.05 ms; 60 primitives hierarchical 8 x 256^2 8.59 -> 0.58 ms; three primitives
+// 2 x 128^2 0.097 -> 0.041 ms; 10 uneven scenes batched 22.8 -> 1.92 ms.
 #include <hip/hip_runtime.h>
 
 #include <algorithm>
