@@ -74,7 +74,7 @@ march_kernel(MarchParams p) {
   RayCounts rc;
   march_ray<PREC, INTEG, 1, B, PREC == PREC_GUARDED && INTEG == INT_SIMPLE && (B == 4 || Q)>(
       p, blockIdx.y, i, j, i < p.res && j < p.res, rc);
-  flush_counts(p, rc);
+  flush_counts<voxel_precision(PREC)>(p, rc);
 }
 
 // Two-pass guarded simple march, first pass: every ray marched without the
@@ -178,7 +178,7 @@ march_hier_redo_kernel(MarchParams p) {
     const int i = (int)(pix / (unsigned)p.res), j = (int)(pix - (unsigned)i * p.res);
     march_ray<PREC_GUARDED, INT_HIERARCHICAL, 1>(p, (int)v, i, j, valid, rc);
   }
-  flush_counts(p, rc);
+  flush_counts<false>(p, rc);
 }
 
 // Resolve pass (two_pass.hpp); the FP64 walks of a root collection visit the
@@ -215,7 +215,7 @@ march_redo_kernel(MarchParams p) {
     const int i = (int)(pix / (unsigned)p.res), j = (int)(pix - (unsigned)i * p.res);
     march_ray<PREC_GUARDED, INT_SIMPLE, 1, B, true>(p, (int)v, i, j, valid, rc);
   }
-  flush_counts(p, rc);
+  flush_counts<false>(p, rc);
 }
 
 // Exact transmittance of listed pixels: item k = (view, i, j) -> vals[k].
@@ -233,7 +233,7 @@ __global__ __launch_bounds__(64) void march_pixels_kernel(MarchParams p, const i
   }
   const double T = march_T<PREC, INTEG, 1>(p, v, i, j, valid, rc);
   if (valid) vals[k] = (float)exp(-T);
-  flush_counts(p, rc);
+  flush_counts<false>(p, rc);
 }
 
 // Exact re-render of listed 16x16 tiles: item k = (view, ti, tj).
@@ -246,7 +246,7 @@ __global__ __launch_bounds__(256) void march_tiles_kernel(MarchParams p, const i
   const int j = it[2] * 16 + (wave & 1) * 8 + (lane & 7);
   RayCounts rc;
   march_ray<PREC, INTEG, 4>(p, it[0], i, j, i < p.res && j < p.res, rc);
-  flush_counts(p, rc);
+  flush_counts<false>(p, rc);
 }
 
 int launch_march_list(const MarchParams& p, int precision, int integrator, const int* items,

@@ -1004,13 +1004,18 @@ __device__ __forceinline__ void march_ray(const MarchParams& p, int v, int i, in
   if (valid) store_pixel(p, v, i, j, T);
 }
 
-// Wave-reduced counters into the launch's counters (lane 0 writes).
+// Wave-reduced counters into the launch's counters (lane 0 writes).  SPREAD:
+// into the block's copy of them.  The sampling marches' waves are few and long
+// and add to the first copy: what the choice of a copy keeps live cost the
+// four-sample form 209 more spilled registers (60 primitives under a
+// sigmoid, 2 x 400^2, step 0.005: 3.28 -> 4.76 ms).
+template <bool SPREAD = true>
 __device__ __forceinline__ void flush_counts(const MarchParams& p, const RayCounts& rc) {
-  unsigned long long* stats = stat_slot(p);
+  unsigned long long* stats = SPREAD ? stat_slot(p) : p.stats;
   if (!stats) return;
-  unsigned long long a = wave_total(rc.samples), b = wave_total(rc.reeval),
-                     c = wave_total(rc.miss), d = wave_total(rc.fine),
-                     e = wave_total(rc.skipped);
+  auto sum = [](unsigned long long v) { return SPREAD ? wave_total(v) : wave_sum(v); };
+  unsigned long long a = sum(rc.samples), b = sum(rc.reeval), c = sum(rc.miss), d = sum(rc.fine),
+                     e = sum(rc.skipped);
   if ((threadIdx.x & 63) == 0) {
     if (a) atomicAdd(stats + ST_SAMPLES, a);
     if (b) atomicAdd(stats + ST_REEVAL, b);
